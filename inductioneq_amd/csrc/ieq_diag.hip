@@ -2,13 +2,14 @@
 // kernel_operator.cl:11-44), the norm of the SBP divergence (calc_div + norm2_S,
 // kernel_operator.cl:98-155) and the error against the testcase's analytic field
 // (analytical_b + norm2_diff, kernel_init.cl:36-48, kernel_operator.cl:50-92), evaluated in
-// one pass with every product and sum in double.  A fixed number of blocks strides over the
-// nodes; each block writes one partial triple and a second one-block kernel adds the
-// partials in a fixed order, so the result is deterministic and independent of the caller.
+// one pass with every product and sum in double.  The blocks split the grid by its sizes alone;
+// each block writes one partial triple and a second one-block kernel adds the partials in a
+// fixed order, so the result is deterministic and independent of the caller.
 #include <mutex>
 
 #include "ieq_device.hpp"
 #include "ieq_diag.hpp"
+#include "ieq_node.hpp"
 
 namespace ieq {
 namespace {
@@ -22,87 +23,159 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch_ptr[kMaxDevices] = {};
 
-template <int OPS>
-__device__ inline double ddiv_dir(const Params& p, const double* hd, int d, uint32_t ix, uint32_t iy, uint32_t iz,
-                                  const float* f32, const double* f64) {
-  using O = Op<OPS>;
-  constexpr int C = (O::W - 1) / 2;
-  const uint32_t n3[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz}, i3[3] = {ix, iy, iz};
-  const int row = bound_row(i3[d], n3[d], O::NB, p.periodic);
-  double acc = 0.0;
-  for (int k = 0; k < O::W; ++k) {
-    const long long j = at_dir(p, ix, iy, iz, d, k - C) + d * p.stride;
-    acc += O::d(row, k) * (f64 ? f64[j] : (double)f32[j]);
-  }
-  return acc / hd[d];
+// Work split of the partial pass: a block takes a run of 256 consecutive nodes of an xy-plane (so the
+// lanes are full whatever nx is) and `zc` planes of it; `segs` runs times `chunks` z-chunks make at most
+// kDiagBlocks blocks.  A plane of more than kDiagBlocks runs is walked with a stride.
+struct DiagSplit {
+  int segs, chunks, zc;
+};
+__host__ __device__ inline DiagSplit diag_split(const Params& p) {
+  const long long nseg = ((long long)p.nx * p.ny + kDiagThreads - 1) / kDiagThreads;
+  DiagSplit s;
+  s.segs = (int)(nseg < kDiagBlocks ? nseg : kDiagBlocks);
+  const int most = kDiagBlocks / s.segs;
+  s.zc = (p.nz + most - 1) / most;
+  s.chunks = (p.nz + s.zc - 1) / s.zc;
+  return s;
 }
 
-template <typename R, int OPS>
-__global__ __launch_bounds__(kDiagThreads) void k_diag(Params p, const R* b, double t, int analytic, double* part) {
+__device__ inline double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// Bound by FP64 instruction issue (about 280 instructions per node with an analytic field) and by the
+// latency of one plane's loads at three waves per SIMD; the node's x and y neighbours are the same for
+// every plane of the chunk, so their rows are found once per thread, and the z row is uniform in a wave.
+// 128^3 FP32, 4th order, with an analytic field: 31 us, against 72 us with a 64-bit division and rolled
+// table rows per node.  TC is the testcase whose analytic field the error is taken against (-1: none):
+// with all of them in one kernel the code of the other seven holds 235 registers (44 us).
+template <typename R, int OPS, int TC>
+__global__ __launch_bounds__(kDiagThreads) void k_diag(Params p, DiagSplit sp, const R* b, double t, double* part) {
   using O = Op<OPS>;
-  const long long n = (long long)p.nx * p.ny * p.nz, S = p.stride, nxy = (long long)p.nx * p.ny;
-  const double hd[3] = {p.dx, p.dy, p.dz};
-  const float* f32 = sizeof(R) == 4 ? (const float*)b : nullptr;
-  const double* f64 = sizeof(R) == 8 ? (const double*)b : nullptr;
+  const int nxy = p.nx * p.ny, per = p.periodic;
+  const long long S = p.stride;
+  const double ih[3] = {1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
+  const int seg0 = (int)blockIdx.x % sp.segs, z0 = ((int)blockIdx.x / sp.segs) * sp.zc, z1 = min(z0 + sp.zc, p.nz);
+  p.testcase = TC;
+  const double st = TC >= 0 ? sin(t) : 0.0, ct = TC >= 0 ? cos(t) : 0.0;
+  __shared__ NodeTable<double, OPS> tab;
+  tab.load(threadIdx.x, kDiagThreads);
+  __syncthreads();
   double acc[3] = {0.0, 0.0, 0.0};
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const uint32_t iz = (uint32_t)(i / nxy), iy = (uint32_t)((i - iz * nxy) / p.nx), ix = (uint32_t)(i - iy * p.nx - iz * nxy);
-    const double fac = (p.dx / O::minv(bound_row(ix, p.nx, O::NB, p.periodic))) *
-                       (p.dy / O::minv(bound_row(iy, p.ny, O::NB, p.periodic))) *
-                       (p.dz / O::minv(bound_row(iz, p.nz, O::NB, p.periodic)));
-    const double bx = (double)b[i], by = (double)b[S + i], bz = (double)b[2 * S + i];
-    acc[0] += fac * (bx * bx + by * by + bz * bz);
-    double dv = 0.0;
-    for (int d = 0; d < 3; ++d) dv += ddiv_dir<OPS>(p, hd, d, ix, iy, iz, f32, f64);
-    acc[1] += fac * (dv * dv);
-    if (analytic) {
-      const V3<double> a = b_analytical<double>(p, ix, iy, iz, t);
-      const double ex = bx - a.x, ey = by - a.y, ez = bz - a.z;
-      acc[2] += fac * (ex * ex + ey * ey + ez * ez);
+  for (int j = seg0 * kDiagThreads + (int)threadIdx.x; j < nxy; j += sp.segs * kDiagThreads) {
+    const int iy = j / p.nx, ix = j - iy * p.nx;
+    const NodeAxis ax = node_axis<OPS>(ix, p.nx, per), ay = node_axis<OPS>(iy, p.ny, per);
+    const bool mxy = __all(ax.mid && ay.mid);
+    const double fxy = (p.dx / O::minv(ax.row)) * (p.dy / O::minv(ay.row));
+    for (int iz = z0; iz < z1; ++iz) {
+      asm volatile("" ::: "memory");  // the table stays in LDS instead of in registers across the planes
+      const NodeAxis az = node_axis<OPS>(iz, p.nz, per);
+      const R* f = b + (long long)iz * nxy;  // plane iz
+      const R *fx = f, *fy = f + S, *fz = f + 2 * S;
+      const double bx = (double)fx[j], by = (double)fy[j], bz = (double)fz[j];
+      const double fac = fxy * (p.dz / O::minv(az.row));
+      acc[0] += fac * (bx * bx + by * by + bz * bz);
+      // one branch for the three directions: the loads of either form are all in flight together
+      double dx, dy, dz;
+      if (mxy && az.mid) {
+        dx = node_deriv_mid<double, OPS>([&](int k) { return (double)fx[j + mid_step(ax, k, per)]; });
+        dy = node_deriv_mid<double, OPS>([&](int k) { return (double)fy[j + p.nx * mid_step(ay, k, per)]; });
+        dz = node_deriv_mid<double, OPS>([&](int k) { return (double)fz[j + (long long)nxy * mid_step(az, k, per)]; });
+      } else {
+        dx = node_deriv_row<double, OPS>(tab, ax, per, [&](int st) { return (double)fx[j + st]; });
+        dy = node_deriv_row<double, OPS>(tab, ay, per, [&](int st) { return (double)fy[j + p.nx * st]; });
+        dz = node_deriv_row<double, OPS>(tab, az, per, [&](int st) { return (double)fz[j + (long long)nxy * st]; });
+      }
+      const double dv = dx * ih[0] + dy * ih[1] + dz * ih[2];
+      acc[1] += fac * (dv * dv);
+      if constexpr (TC >= 0) {
+        const V3<double> a = b_analytical<double>(p, ix, iy, iz, t, st, ct);
+        const double ex = bx - a.x, ey = by - a.y, ez = bz - a.z;
+        acc[2] += fac * (ex * ex + ey * ey + ez * ez);
+      }
     }
   }
-  __shared__ double sm[3][kDiagThreads];
-  for (int c = 0; c < 3; ++c) sm[c][threadIdx.x] = acc[c];
-  __syncthreads();
-  for (int s = kDiagThreads / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s)
-      for (int c = 0; c < 3; ++c) sm[c][threadIdx.x] += sm[c][threadIdx.x + s];
-    __syncthreads();
+  __shared__ double sm[3][kDiagThreads / 64];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double v = wave_sum(acc[c]);
+    if ((threadIdx.x & 63) == 0) sm[c][threadIdx.x >> 6] = v;
   }
-  if (threadIdx.x < 3) part[blockIdx.x * 3 + threadIdx.x] = sm[threadIdx.x][0];
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double s = 0.0;
+    for (int w = 0; w < kDiagThreads / 64; ++w) s += sm[threadIdx.x][w];
+    part[blockIdx.x * 3 + threadIdx.x] = s;
+  }
 }
 
-// out = (energy, divergence norm, error norm) from nblk partial triples, summed in block order;
-// the error norm is NaN without an analytic field.
-__global__ __launch_bounds__(64) void k_diag_sum(const double* part, int nblk, int analytic, double* out) {
+// out = (energy, divergence norm, error norm) from nblk partial triples, summed in a fixed order by one
+// workgroup (three lanes adding 1024 triples one after the other took 107 us); the error norm is NaN
+// without an analytic field.
+__global__ __launch_bounds__(kDiagThreads) void k_diag_sum(const double* part, int nblk, int analytic, double* out) {
+  __shared__ double sm[3][kDiagThreads / 64];
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int k = threadIdx.x; k < nblk; k += kDiagThreads)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[c] += part[k * 3 + c];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double v = wave_sum(acc[c]);
+    if ((threadIdx.x & 63) == 0) sm[c][threadIdx.x >> 6] = v;
+  }
+  __syncthreads();
   if (threadIdx.x >= 3) return;
   double s = 0.0;
-  for (int k = 0; k < nblk; ++k) s += part[k * 3 + threadIdx.x];
+  for (int w = 0; w < kDiagThreads / 64; ++w) s += sm[threadIdx.x][w];
   out[threadIdx.x] = threadIdx.x == 0 ? s : (threadIdx.x == 2 && !analytic) ? __longlong_as_double(0x7ff8000000000000LL)
                                                                             : sqrt(fmax(s, 0.0));
+}
+
+template <typename R, int OPS> const void* diag_kernel_t(int tc) {
+  switch (tc) {
+    case TC_ROTATION_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_2D>);
+    case TC_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_3D>);
+    case TC_HALL_PERIODIC: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_PERIODIC>);
+    case TC_HALL_TRAVELLING_WAVE: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_TRAVELLING_WAVE>);
+    case TC_CONFINED_DOMAIN: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_CONFINED_DOMAIN>);
+    case TC_ALFVEN_PERIODIC_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ALFVEN_PERIODIC_2D>);
+    case TC_GAUSSIAN_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_GAUSSIAN_ROTATION_3D>);
+    case TC_UNIFORM_FLOW: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_UNIFORM_FLOW>);
+    default: return reinterpret_cast<const void*>(&k_diag<R, OPS, -1>);
+  }
+}
+template <typename R> const void* diag_kernel(int ops, int tc) {
+  switch (ops) {
+    case 0: return diag_kernel_t<R, 0>(tc);
+    case 1: return diag_kernel_t<R, 1>(tc);
+    case 2: return diag_kernel_t<R, 2>(tc);
+    case 3: return diag_kernel_t<R, 3>(tc);
+    case 4: return diag_kernel_t<R, 4>(tc);
+    default: return diag_kernel_t<R, 5>(tc);
+  }
 }
 
 }  // namespace
 
 int diag_blocks(const Params& p) {
-  const long long n = (long long)p.nx * p.ny * p.nz;
-  const long long need = (n + kDiagThreads - 1) / kDiagThreads;
-  return (int)(need < kDiagBlocks ? need : kDiagBlocks);
+  const DiagSplit s = diag_split(p);
+  return s.segs * s.chunks;
 }
 
 template <typename R>
 hipError_t diag_launch(const Params& p, int ops, hipStream_t s, const R* b, double t, int analytic, double* part,
                        double* out_dev) {
-  const int nblk = diag_blocks(p);
-  switch (ops) {
-    case 0: k_diag<R, 0><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-    case 1: k_diag<R, 1><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-    case 2: k_diag<R, 2><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-    case 3: k_diag<R, 3><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-    case 4: k_diag<R, 4><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-    default: k_diag<R, 5><<<nblk, kDiagThreads, 0, s>>>(p, b, t, analytic, part); break;
-  }
-  k_diag_sum<<<1, 64, 0, s>>>(part, nblk, analytic, out_dev);
+  const DiagSplit sp = diag_split(p);
+  const int nblk = sp.segs * sp.chunks;
+  const void* k = diag_kernel<R>(ops, analytic ? p.testcase : -1);
+  Params q = p;
+  DiagSplit split = sp;
+  void* kargs[5] = {(void*)&q, (void*)&split, (void*)&b, (void*)&t, (void*)&part};
+  const hipError_t e = hipLaunchKernel(k, dim3(nblk), dim3(kDiagThreads), kargs, 0, s);
+  if (e != hipSuccess) return e;
+  k_diag_sum<<<1, kDiagThreads, 0, s>>>(part, nblk, analytic, out_dev);
   return hipGetLastError();
 }
 
