@@ -18,6 +18,7 @@
 #include "ieq_diag.hpp"
 #include "ieq_fused.hpp"
 #include "ieq_generic.hpp"
+#include "ieq_node_stage.hpp"
 #include "ieq_tiled.hpp"
 
 using ieq::Params;
@@ -172,8 +173,8 @@ struct ieq_program {
   ieq::FusedWork* fused = nullptr;
   ieq::CgWork* cg = nullptr;
   int last_path = -1;  // path of the last ieq_run / ieq_step: 0 reference kernels, 1 fused kernels, 2 reference
-                       // sequence with the tiled stage kernel
-  bool tiled_used = false;  // the current ieq_run / ieq_step launched a tiled stage
+                       // sequence with whole-grid stages of a program the tiled kernel covers
+  bool tiled_used = false;  // the current ieq_run / ieq_step launched such a stage
   double* diag = nullptr;  // ieq_diagnostics: 3 * kDiagBlocks partials + the 3 results
 
   bool has(const char* m) const { return modules.count(m) != 0; }
@@ -404,15 +405,17 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
       case K_STAGE: {
         R* P = st->P >= 0 ? F[st->P] : nullptr;
         R* Q = st->Q >= 0 ? F[st->Q] : nullptr;
-        // the whole grid of a program the tiled kernel covers: z-marching tiles; otherwise (or for
-        // a part of the grid) one work-item per node
-        if (full_grid(pr, g) && ieq::tiled_stage_ok(p, ops, (int)sizeof(R))) {
-          hipError_t e = ieq::tiled_stage<R>(p, ops, s, F[st->out], P, (R)st->cP, Q, (R)st->cQ, F[st->Y], (R)(st->cD * p.dt), u, time);
-          if (e != hipSuccess) return hip_fail(pr, e, name);
-          pr->tiled_used = true;
-        } else {
-          ieq::gen_stage<R>(p, ops, s, g, F[st->out], P, (R)st->cP, Q, (R)st->cQ, F[st->Y], (R)(st->cD * p.dt), J, u, time);
-        }
+        // the whole grid of a program the tiled kernel covers: z-marching tiles where they are the faster
+        // kernel; otherwise (or for a part of the grid) a thread per node
+        const bool whole = full_grid(pr, g) && ieq::tiled_stage_ok(p, ops, (int)sizeof(R));
+        hipError_t e;
+        if (whole && ieq::tiled_stage_pays(p, ops, (int)sizeof(R)))
+          e = ieq::tiled_stage<R>(p, ops, s, F[st->out], P, (R)st->cP, Q, (R)st->cQ, F[st->Y], (R)(st->cD * p.dt), u, time);
+        else
+          e = ieq::node_stage<R>(p, ops, s, g, F[st->out], P, (R)st->cP, Q, (R)st->cQ, F[st->Y], (R)(st->cD * p.dt), J, u,
+                                 ieq::NodeTime<R>{time});
+        if (e != hipSuccess) return hip_fail(pr, e, name);
+        if (whole) pr->tiled_used = true;
         break;
       }
       case K_2R:
@@ -431,11 +434,13 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
         ieq::gen_time<R>(s, time, 0, p.dt, 1);
         break;
       case K_U:
-        ieq::gen_calc_u<R>(p, s, g, u, time);
+      case K_CURL: {
+        const bool c = st->kind == K_CURL;
+        hipError_t e = ieq::node_pre<R>(p, ops, s, g, c ? F[st->Y] : nullptr, c ? J : nullptr, rho, c ? nullptr : u,
+                                        ieq::NodeTime<R>{time});
+        if (e != hipSuccess) return hip_fail(pr, e, name);
         break;
-      case K_CURL:
-        ieq::gen_curl_rho<R>(p, ops, s, g, F[st->Y], J, rho);
-        break;
+      }
     }
     return IEQ_OK;
   }

@@ -80,9 +80,9 @@ __global__ __launch_bounds__(kDiagThreads) void k_diag(Params p, DiagSplit sp, c
       // one branch for the three directions: the loads of either form are all in flight together
       double dx, dy, dz;
       if (mxy && az.mid) {
-        dx = node_deriv_mid<double, OPS>([&](int k) { return (double)fx[j + mid_step(ax, k, per)]; });
-        dy = node_deriv_mid<double, OPS>([&](int k) { return (double)fy[j + p.nx * mid_step(ay, k, per)]; });
-        dz = node_deriv_mid<double, OPS>([&](int k) { return (double)fz[j + (long long)nxy * mid_step(az, k, per)]; });
+        dx = node_deriv_mid<double, OPS>([&](int k) { return (double)fx[j + node_step(ax, k, per)]; });
+        dy = node_deriv_mid<double, OPS>([&](int k) { return (double)fy[j + p.nx * node_step(ay, k, per)]; });
+        dz = node_deriv_mid<double, OPS>([&](int k) { return (double)fz[j + (long long)nxy * node_step(az, k, per)]; });
       } else {
         dx = node_deriv_row<double, OPS>(tab, ax, per, [&](int st) { return (double)fx[j + st]; });
         dy = node_deriv_row<double, OPS>(tab, ay, per, [&](int st) { return (double)fy[j + p.nx * st]; });

@@ -25,6 +25,7 @@
 #include "ieq_fused_tiles.hpp"
 #include "ieq_generic.hpp"
 #include "ieq_hall.hpp"
+#include "ieq_node_stage.hpp"
 #include "ieq_stencil.hpp"
 
 namespace ieq {
@@ -638,7 +639,8 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     // curlB_rho as the reference schedule leaves it: calc_curlB_rho of the last stage's input
     // (still intact: a register of the 3-register schemes, the ping-pong copy of the 2N ones)
     const uint32_t g[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz};
-    gen_curl_rho<R>(p, info.opset, s, g, y_last, J, rho);
+    const hipError_t e = node_pre<R>(p, info.opset, s, g, y_last, J, rho, (R*)nullptr, NodeTime<R>());
+    if (e != hipSuccess) return err = std::string("fused launch: ") + hipGetErrorString(e), IEQ_ERR_HIP;
   }
   if (b1 != F[0]) {
     if (hipMemcpyAsync(F[0], b1, vbytes, hipMemcpyDeviceToDevice, s) != hipSuccess) return err = "copy-back failed", IEQ_ERR_HIP;

@@ -10,147 +10,6 @@ namespace {
 
 constexpr int BX = 64, BY = 4;
 
-// kappa4 of include/artificial_dissipation.h:23-45 (k enters only through k*k).
-template <typename R>
-__device__ inline V3<R> kappa3(const Params& p, uint32_t k, R h, V3<R> b1, V3<R> b2, V3<R> u1, V3<R> u2) {
-  k = k + (k == 0u);
-  R kk = (R)(uint32_t)(k * k);
-  R lo = kk * (R)p.mp2min * (R)p.cmin * h, hi = kk * (R)p.mp2max * (R)p.cmax * h;
-  R out[3];
-  for (int c = 0; c < 3; ++c) {
-    R db = cmp(b1, c) - cmp(b2, c);
-    R s = fmax(fabs(cmp(u1, c)), fabs(cmp(u2, c))) * db * db;
-    out[c] = (R)((lo < s) && (s < hi)) * sqrt(fabs(s - lo) / fabs(hi - lo)) + (R)(s >= hi);
-  }
-  return {out[0], out[1], out[2]};
-}
-
-// One HOD partial sum, diff_HOD_* of include/artificial_dissipation.h:58-101.
-template <typename R, int OPS>
-__device__ inline V3<R> hod_part(const Params& p, const R* b, uint32_t ix, uint32_t iy, uint32_t iz, int d, int row, int s) {
-  using O = Op<OPS>;
-  const long long S = p.stride;
-  const R sgn = ((O::ORDER / 2 + 1) & 1) ? R(-1) : R(1);
-  V3<R> h = zero3<R>();
-  for (int i = 0; i < O::WH; ++i) {
-    R coef = (R)O::minv(row) * (R)O::dho(row, s + O::WH - 1) * (R)O::dho(O::NB, i) * sgn;
-    h = h + coef * ld3(b, S, at_dir(p, ix, iy, iz, d, i + s));
-  }
-  return h;
-}
-
-// The semi-discrete right-hand side DB (kernel_time_integrator.cl:9-31).
-template <typename R, int OPS>
-__device__ V3<R> rhs_node(const Params& p, uint32_t ix, uint32_t iy, uint32_t iz, const R* b, const R* J, const R* u, R t) {
-  using O = Op<OPS>;
-  constexpr int C = (O::W - 1) / 2;
-  const long long S = p.stride;
-  const long long i0 = lin(p, ix, iy, iz);
-  const uint32_t n3[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz}, i3[3] = {ix, iy, iz};
-  int rows[3];
-  for (int d = 0; d < 3; ++d) rows[d] = bound_row(i3[d], n3[d], O::NB, p.periodic);
-
-  // convec_volume: induction_Eq_volume.cl:168-212
-  V3<R> Bm = ld3(b, S, i0), um = ld3(u, S, i0);
-  V3<R> db = zero3<R>();
-  for (int d = 0; d < 3; ++d) {
-    V3<R> acc = zero3<R>();
-    for (int i = 0; i < O::W; ++i) {
-      R c = (R)O::d(rows[d], i);
-      long long j = at_dir(p, ix, iy, iz, d, i - C);
-      acc = acc + c * volume_flux(p, d, Bm, um, ld3(b, S, j), ld3(u, S, j));
-    }
-    db = db + (R)(2.0 / hdir(p, d)) * acc;
-  }
-
-  const R m0 = (R)O::minv(0);
-  if (p.hall) {
-    if (!p.periodic) {  // convec_Hall_surface: induction_Eq_surface.cl:35-81
-      V3<R> Jc = ld3(J, S, i0);
-      V3<R> tv = R(0.5) * um - Jc;
-      V3<R> sat = zero3<R>();
-      for (int d = 0; d < 3; ++d) {
-        int l = i3[d] == 0, r = i3[d] == n3[d] - 1;
-        R tvd = cmp(tv, d);
-        R s1 = (R)(l * (tvd > R(0))) * R(-1) + (R)(r * (tvd < R(0)));
-        R s2 = (R)l * R(-1) + (R)r;
-        sat = sat + (R)(m0 / (R)hdir(p, d)) * ((s1 * tvd) * Bm + (s2 * cmp(Bm, d)) * Jc);
-      }
-      db = db + sat;
-    }
-    // Hall_volume: induction_Eq_volume.cl:215-256
-    V3<R> hv = zero3<R>();
-    for (int d = 0; d < 3; ++d) {
-      V3<R> acc = zero3<R>();
-      for (int i = 0; i < O::W; ++i) {
-        R c = (R)O::d(rows[d], i);
-        long long j = at_dir(p, ix, iy, iz, d, i - C);
-        V3<R> B = ld3(b, S, j), Jk = ld3(J, S, j);
-        acc = acc + c * (cmp(Jk, d) * B - cmp(B, d) * Jk);
-      }
-      hv = hv + (R)(1.0 / hdir(p, d)) * acc;
-    }
-    db = db + hv;
-  } else if (!p.periodic) {  // convec_surface: induction_Eq_surface.cl:7-33
-    V3<R> g = b_boundary<R>(p, ix, iy, iz, t);
-    V3<R> diff = Bm - g;
-    V3<R> sat = zero3<R>();
-    for (int d = 0; d < 3; ++d) {
-      R ud = cmp(um, d);
-      R s = (R)((i3[d] == 0) * (ud > R(0))) * R(-1) + (R)((i3[d] == n3[d] - 1) * (ud < R(0)));
-      sat = sat + ((R)(m0 / (R)hdir(p, d)) * s * ud) * diff;
-    }
-    db = db + sat;
-  }
-
-  if (p.diss == 1) {  // high_order_dissipation: artificial_dissipation.cl:13-32
-    const R F = (R)p.ho_factor;
-    V3<R> h = zero3<R>();
-    for (int s = -O::WH + 1; s < 1; ++s)
-      for (int d = 0; d < 3; ++d) h = h + F * hod_part<R, OPS>(p, b, ix, iy, iz, d, rows[d], s);
-    db = db + h;
-  } else if (p.diss == 2) {  // first_order_dissipation: artificial_dissipation.cl:36-79
-    V3<R> fo = zero3<R>();
-    for (int d = 0; d < 3; ++d) {
-      V3<R> acc = zero3<R>();
-      for (int i = 0; i < O::W; ++i) {
-        long long j = at_dir(p, ix, iy, iz, d, i - C);
-        V3<R> sg = sigma3(ld3(u, S, j), um), dB = ld3(b, S, j) - Bm;
-        R c = (R)fabs(O::d(rows[d], i));
-        acc = acc + mk(c * sg.x * dB.x, c * sg.y * dB.y, c * sg.z * dB.z);
-      }
-      R h = (R)hdir(p, d);
-      fo = fo + mk(acc.x / h, acc.y / h, acc.z / h);
-    }
-    db = db + fo;
-  } else if (p.diss == 3) {  // adaptive_dissipation: artificial_dissipation.cl:83-160
-    V3<R> ad = zero3<R>();
-    for (int d = 0; d < 3; ++d) {
-      R h = (R)hdir(p, d);
-      V3<R> acc = zero3<R>();
-      for (int i = 0; i < O::W; ++i) {
-        long long j = at_dir(p, ix, iy, iz, d, i - C);
-        V3<R> Bk = ld3(b, S, j), uk = ld3(u, S, j);
-        V3<R> kap = kappa3<R>(p, (uint32_t)i - (uint32_t)C, h, Bk, Bm, uk, um);
-        V3<R> sg = sigma3(uk, um), dB = Bk - Bm;
-        R c = (R)fabs(O::d(rows[d], i));
-        acc = acc + mk(c * kap.x * sg.x * dB.x, c * kap.y * sg.y * dB.y, c * kap.z * sg.z * dB.z);
-      }
-      ad = ad + mk(acc.x / h, acc.y / h, acc.z / h);
-    }
-    const R F = (R)p.ho_factor;
-    for (int s = -O::WH + 1; s <= 0; ++s)
-      for (int d = 0; d < 3; ++d) {
-        long long j1 = at_dir(p, ix, iy, iz, d, s + O::WH - 1), j2 = at_dir(p, ix, iy, iz, d, s + O::WH - 2);
-        V3<R> kap = kappa3<R>(p, 1u, (R)hdir(p, d), ld3(b, S, j1), ld3(b, S, j2), ld3(u, S, j1), ld3(u, S, j2));
-        V3<R> hp = hod_part<R, OPS>(p, b, ix, iy, iz, d, rows[d], s);
-        ad = ad + mk((R(1) - kap.x) * F * hp.x, (R(1) - kap.y) * F * hp.y, (R(1) - kap.z) * F * hp.z);
-      }
-    db = db + ad;
-  }
-  return db;
-}
-
 // d/dx_d of a vector field (diff_x/y/z, SBP_operator.cl:12-51) or of its M-adjoint.
 template <typename R, int OPS, bool ADJ>
 __device__ inline V3<R> dvec(const Params& p, const R* f, uint32_t ix, uint32_t iy, uint32_t iz, int d) {
@@ -196,19 +55,6 @@ template <typename R, int OPS> __device__ inline R div_node(const Params& p, con
   (void)S; (void)idx;
 
 struct Range { uint32_t x, y, z; };
-
-// out = cP*P + cQ*Q + cD*DB(Y); null P/Q contribute nothing.
-template <typename R, int OPS>
-__global__ __launch_bounds__(BX* BY) void k_stage(Params p, Range g, R* out, const R* P, R cP, const R* Q, R cQ, const R* Y,
-                                                  R cD, const R* J, const R* u, const R* time) {
-  IEQ_NODE_PREAMBLE(0)
-  const R t = time[1];
-  V3<R> d = rhs_node<R, OPS>(p, ix, iy, iz, Y, J, u, t);
-  V3<R> r = cD * d;
-  if (Q) r = cQ * ld3(Q, S, idx) + r;
-  if (P) r = cP * ld3(P, S, idx) + r;
-  st3(out, S, idx, r);
-}
 
 template <typename R> __device__ inline void set_time(const Range& g, R* time, double c, double dt, uint32_t ix, uint32_t iy, uint32_t iz) {
   if (ix == 0 && iy == 0 && iz == 0 && c >= 0) time[1] = time[0] + (R)c * (R)dt;
@@ -256,19 +102,6 @@ template <typename R> __global__ void k_time(R* time, double c, double dt, int m
       time[1] = time[0] + (R)(c * dt);
     }
   }
-}
-
-template <typename R, int OPS>
-__global__ __launch_bounds__(BX* BY) void k_curl_rho(Params p, Range g, const R* b, R* J, const R* rho) {
-  IEQ_NODE_PREAMBLE(0)
-  V3<R> c = curl_node<R, OPS>(p, b, ix, iy, iz);
-  R r = rho[idx];
-  st3(J, S, idx, mk(c.x / r, c.y / r, c.z / r));
-}
-
-template <typename R> __global__ __launch_bounds__(BX* BY) void k_calc_u(Params p, Range g, R* u, const R* time) {
-  IEQ_NODE_PREAMBLE(0)
-  st3(u, S, idx, u_analytical<R>(p, ix, iy, iz, time[1]));
 }
 
 // init_b / init_u / init_rho / analytical_b (kernel_init.cl:3-48)
@@ -424,13 +257,6 @@ dim3 grid_of(Range g) { return dim3((g.x + BX - 1) / BX, (g.y + BY - 1) / BY, g.
   }
 
 template <typename R>
-void gen_stage(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* out, const R* P, R cP, const R* Q, R cQ,
-               const R* Y, R cD, const R* J, const R* u, const R* time) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_stage<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, out, P, cP, Q, cQ, Y, cD, J, u, time)))
-}
-
-template <typename R>
 void gen_update_2r(const Params& p, hipStream_t s, const uint32_t g[3], R* X, R* O, const R* D, R a, R b, R* time, double tc) {
   Range r{g[0], g[1], g[2]};
   k_update_2r<R><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, X, O, D, a, b, time, tc);
@@ -449,16 +275,6 @@ template <typename R> void gen_ssprk104_06(const Params& p, hipStream_t s, const
 
 template <typename R> void gen_time(hipStream_t s, R* time, double c, double dt, int mode) {
   k_time<R><<<1, 64, 0, s>>>(time, c, dt, mode);
-}
-
-template <typename R> void gen_curl_rho(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* J, const R* rho) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_curl_rho<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, b, J, rho)))
-}
-
-template <typename R> void gen_calc_u(const Params& p, hipStream_t s, const uint32_t g[3], R* u, const R* time) {
-  Range r{g[0], g[1], g[2]};
-  k_calc_u<R><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, u, time);
 }
 
 template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32_t g[3], R* f, int which, const R* time) {
@@ -510,14 +326,10 @@ template <typename R> void gen_soa_to_aos(hipStream_t s, const R* soa, R* aos, l
 }
 
 #define IEQ_INSTANTIATE(R)                                                                                                   \
-  template void gen_stage<R>(const Params&, int, hipStream_t, const uint32_t*, R*, const R*, R, const R*, R, const R*, R,  \
-                             const R*, const R*, const R*);                                                                  \
   template void gen_update_2r<R>(const Params&, hipStream_t, const uint32_t*, R*, R*, const R*, R, R, R*, double);           \
   template void gen_update_2n<R>(const Params&, hipStream_t, const uint32_t*, R*, const R*, R, R*, double);                  \
   template void gen_ssprk104_06<R>(const Params&, hipStream_t, const uint32_t*, const R*, R*, R*, R*);                        \
   template void gen_time<R>(hipStream_t, R*, double, double, int);                                                           \
-  template void gen_curl_rho<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*, const R*);                   \
-  template void gen_calc_u<R>(const Params&, hipStream_t, const uint32_t*, R*, const R*);                                    \
   template void gen_init<R>(const Params&, hipStream_t, const uint32_t*, R*, int, const R*);                                 \
   template void gen_div<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*, int);                             \
   template void gen_curl<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                 \

@@ -28,15 +28,11 @@ template <int OPS> __device__ __forceinline__ NodeAxis node_axis(int i, int n, i
   a.mid = a.row == O::NB && (periodic || (i >= RR && i + RR < n));
   return a;
 }
-// Position along the axis of the neighbour at offset k of a mid node, relative to the node.
-__device__ __forceinline__ int mid_step(const NodeAxis& a, int k, int periodic) {
-  int j = a.i + k;
-  if (periodic) j += j < 0 ? a.n : j >= a.n ? -a.n : 0;
-  return j - a.i;
-}
-// The same for any node: a neighbour outside a bounded grid is the node itself.
-__device__ __forceinline__ int any_step(const NodeAxis& a, int k, int periodic) {
-  return (int)nbr((uint32_t)a.i, k, (uint32_t)a.n, periodic) - a.i;
+// Step along the axis to the neighbour at offset k: wrapped on periodic grids; a neighbour outside a
+// bounded grid is the node itself.  Without branches, so that the loads that follow stay in one run.
+__device__ __forceinline__ int node_step(const NodeAxis& a, int k, int periodic) {
+  const int out = periodic ? (k < 0 ? k + a.n : k - a.n) : 0;
+  return (unsigned)(a.i + k) < (unsigned)a.n ? k : out;
 }
 
 // Value at a byte offset from a component's base; I is unsigned where three components of a field
@@ -70,7 +66,7 @@ __device__ __forceinline__ T node_deriv_row(const NodeTable<T, OPS>& t, const No
   constexpr int W = NodeTable<T, OPS>::W, C = NodeTable<T, OPS>::C;
   T acc = T(0);
 #pragma unroll
-  for (int k = 0; k < W; ++k) acc = acc + t.c[a.row][k] * at(any_step(a, k - C, periodic));
+  for (int k = 0; k < W; ++k) acc = acc + t.c[a.row][k] * at(node_step(a, k - C, periodic));
   return acc;
 }
 

@@ -16,6 +16,9 @@ struct Params;
 // the stencil width, 32-bit byte offsets for three component planes.
 bool tiled_stage_ok(const Params& p, int ops, int real_bytes);
 
+// Whether the tiled kernel is the faster one for such a program, or a thread per node (node_stage).
+bool tiled_stage_pays(const Params& p, int ops, int real_bytes);
+
 // Enqueue one stage on the whole grid: out = cP*P + cQ*Q + cD*DB(Y) (P or Q null: absent), the
 // velocity field u, the stage time read from time[1] on the device, as the reference stage does.
 template <typename R>

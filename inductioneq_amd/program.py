@@ -194,7 +194,8 @@ class Program:
     @property
     def last_step_path(self) -> str:
         """Path of the last run / step call (ieq_last_step_path): "fused", "tiled" (the reference kernel
-        sequence with the z-marching stage kernel), "reference" (one work-item per node) or "none"."""
+        sequence on the whole grid of a program the z-marching stage kernel covers, which small grids run with a
+        thread per node), "reference" (a thread per node) or "none"."""
         return {1: "fused", 2: "tiled", 0: "reference"}.get(self.lib.ieq_last_step_path(self.handle), "none")
 
     def reduce(self, name: str, *fields) -> float:

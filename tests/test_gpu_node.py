@@ -36,3 +36,73 @@ def test_diagnostics_split(ops, n, per, tc, real):
     want = _oracle_diag(cfg, B, 0.2)
     for g, w in zip((got["energy"], got["divergence_norm"], got["error_norm"]), want):
         assert abs(g - w) <= 1e-12 * abs(w), (got, want)
+
+
+def _stage_case(ops, n, per, hall, diss, real, seed=11):
+    from test_gpu_tiled import FORMS, _cfg, _fields
+
+    cfg = _cfg(ops, n, per, diss, FORMS[seed % len(FORMS)], "hall_periodic" if hall else "rotation_2D", real)
+    cfg.hall = hall
+    B, U = _fields(cfg, seed)
+    return cfg, B, U
+
+
+@pytest.mark.parametrize("ops,n,per,hall,diss,real", [
+    ("4thOrder", (13, 5, 9), False, True, None, "double"),             # a run of 64 nodes and one of 1; y within two closures
+    ("6thOrder", (8, 8, 7), False, True, "HIGH_ORDER", "double"),      # runs of exactly 64, boundary rows in every direction
+    ("6thOrderExtended", (70, 16, 15), False, True, "ADAPTIVE", "double"),
+    ("2ndOrderExtended", (5, 30, 6), True, True, "FIRST_ORDER", "double"),
+    ("4thOrderExtended", (12, 11, 65), False, False, "ADAPTIVE", "float"),
+    ("6thOrder", (130, 11, 10), True, False, "HIGH_ORDER", "float"),     # periodic, runs across row ends
+    ("2ndOrder", (2, 20, 18), False, True, None, "double"),            # two nodes in x
+    ("6thOrderExtended", (64, 8, 17), False, False, "FIRST_ORDER", "float"),  # y as narrow as the reference reads in bounds
+])
+@pytest.mark.parametrize("part", [False, True])
+def test_node_kernels_equal_oracle(ops, n, per, hall, diss, real, part):
+    """calc_curlB_rho, calc_u and the two kinds of stage (SSPRK33_3b: two operands; CarpenterKennedy2N54_2a: in
+    place) against the oracle, on the whole grid and on a part of it whose other nodes stay as they were.
+    FP64 1e-12 of the largest value (sums of at most 3 x 15 x 9 products), FP32 2e-5."""
+    import os
+
+    import torch
+    from pyoracle import Oracle
+
+    from inductioneq_amd.program import Program
+    from test_gpu_tiled import TOL, _aos
+
+    cfg, B, U = _stage_case(ops, n, per, hall, diss, real)
+    g = tuple(max(1, v - 1 - k) for k, v in enumerate(n)) if part else n
+    prog, orc = Program(cfg), Oracle(cfg)
+    rng = np.random.default_rng(4)
+    regs = [_aos(cfg, B + 0.1 * rng.standard_normal(B.shape)) for _ in range(3)]
+    rho = (1.0 + 0.2 * rng.random(cfg.num_nodes_pad)).astype(cfg.dtype)
+    os.environ["IEQ_NO_TILED"] = "1"
+    try:
+        for names, nf in ((["calc_curlB_rho_3_3args", "calc_u_3_args", "SSPRK33_3b"], 3),
+                          (["calc_curlB_rho_1_2args", "CarpenterKennedy2N54_2a"], 2)):
+            names = [k for k in names if hall or not k.startswith("calc_curlB")]
+            host = [r.copy() for r in regs[:nf]] + [orc.vec(), _aos(cfg, U), rho.copy(), orc.time(0.3)]
+            dev = [prog.upload_real4(a) for a in host[: nf + 2]] + [prog.upload_real(host[nf + 2])]
+            dev.append(torch.tensor([0.3, 0.3], dtype=prog.torch_dtype, device="cuda"))
+            for k in names:
+                orc.run(k, host, g=g)
+                prog.run(k, dev, g=g)
+            for i in range(nf + 2):
+                got = prog.download_real4(dev[i])[: cfg.num_nodes, :3].astype(np.float64)
+                want = host[i][: cfg.num_nodes, :3].astype(np.float64)
+                e = np.abs(got - want).max() / max(np.abs(want).max(), 1e-300)
+                assert e <= TOL[real], (names, i, e)
+    finally:
+        os.environ.pop("IEQ_NO_TILED", None)
+
+
+@pytest.mark.parametrize("ops", ["2ndOrder", "4thOrder", "6thOrder", "2ndOrderExtended", "4thOrderExtended", "6thOrderExtended"])
+@pytest.mark.parametrize("diss,real", [(None, "double"), ("HIGH_ORDER", "float"), ("FIRST_ORDER", "double")])
+def test_tiled_stage_on_small_grids(ops, diss, real):
+    """The z-marching kernel where a thread per node would be taken (a stated z-chunk keeps the tiles)."""
+    from test_gpu_tiled import FORMS, _cfg, _check, _run_both
+
+    cfg = _cfg(ops, (37, 21, 19), False, diss, FORMS[2], "rotation_2D", real)
+    prog, db, hb, path = _run_both(cfg, "SSPRK33", env={"IEQ_TILED_ZC": "4"})
+    assert path == "tiled"
+    _check(cfg, prog, db, hb, "SSPRK33", "%s %s" % (ops, diss))
