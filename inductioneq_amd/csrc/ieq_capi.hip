@@ -9,6 +9,8 @@
 #include <map>
 #include <set>
 #include <string>
+#include <string_view>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/inductioneq.h"
@@ -148,9 +150,13 @@ const StageDesc kStages[] = {
 #undef CK
 
 const StageDesc* find_stage(const char* name) {
-  for (const auto& s : kStages)
-    if (!std::strcmp(s.name, name)) return &s;
-  return nullptr;
+  static const std::unordered_map<std::string_view, const StageDesc*> by_name = [] {
+    std::unordered_map<std::string_view, const StageDesc*> m;
+    for (const auto& s : kStages) m.emplace(s.name, &s);
+    return m;
+  }();
+  const auto it = by_name.find(name);
+  return it == by_name.end() ? nullptr : it->second;
 }
 
 std::string module_base(const char* m) {
@@ -176,6 +182,11 @@ struct ieq_program {
                        // sequence with whole-grid stages of a program the tiled kernel covers
   bool tiled_used = false;  // the current ieq_run / ieq_step launched such a stage
   double* diag = nullptr;  // ieq_diagnostics: 3 * kDiagBlocks partials + the 3 results
+  // second copy of b1 for 2N stages that update it in the stage kernel (neighbours still read the first),
+  // the stream whose launches used it last and their end
+  void* b1_copy = nullptr;
+  hipStream_t b1_copy_stream = nullptr;
+  hipEvent_t b1_copy_done = nullptr;
 
   bool has(const char* m) const { return modules.count(m) != 0; }
   int fail(int code, const std::string& msg) {
@@ -497,17 +508,137 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
   return pr->fail(IEQ_ERR_KERNEL, std::string("kernel not in program: ") + name);
 }
 
+// The second copy of b1, ordered after its last use; null where it cannot be had: no memory, or the stream is
+// being captured (an allocation or a wait on another stream's event would end the capture, and a replay would
+// share the buffer with calls it is not ordered with).
+void* b1_copy_for(ieq_program* pr) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(pr->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
+  if (!pr->b1_copy_done && hipEventCreateWithFlags(&pr->b1_copy_done, hipEventDisableTiming) != hipSuccess) {
+    pr->b1_copy_done = nullptr;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (!pr->b1_copy) {
+    const size_t bytes = (size_t)3 * pr->info.stride * pr->info.real_bytes;
+    if (hipMalloc(&pr->b1_copy, bytes) != hipSuccess) {
+      pr->b1_copy = nullptr;
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    pr->b1_copy_stream = pr->stream;
+  } else if (pr->b1_copy_stream != pr->stream) {
+    if (hipStreamWaitEvent(pr->stream, pr->b1_copy_done, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    pr->b1_copy_stream = pr->stream;
+  }
+  return pr->b1_copy;
+}
+
+// Runs a kernel list.  Neighbouring kernels of the time integrators share a launch where every kernel of the
+// group would be accepted by itself and no value differs: calc_curlB_rho + calc_u; a kernel that only sets the
+// stage time and the kernel that reads it; and, on the whole grid, the two halves of a 2N stage (b1' goes to a
+// second copy of b1, in pairs, so that b1 ends where it began).
+template <typename R>
+int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t g[3], const uint32_t l[3], void* const* args,
+               int nargs) {
+  const Params& p = pr->p;
+  const int ops = pr->info.opset;
+  hipStream_t s = pr->stream;
+  std::vector<void*> A(args, args + std::max(nargs, 0));
+  bool all_set = true;
+  for (void* a : A) all_set = all_set && a != nullptr;
+  const bool modules = pr->has("kernel_time_integrator"), rhs = pr->has("induction_Eq_volume") && pr->has("induction_Eq_surface");
+  const bool in_range = range_ok(pr, g, 0), whole = full_grid(pr, g);
+  auto accepted = [&](const char* name) -> const StageDesc* {  // a time-integrator kernel that run_one would launch
+    const StageDesc* st = name ? find_stage(name) : nullptr;
+    return st && all_set && modules && (rhs || st->kind != K_STAGE) && nargs == st->nf + 4 && in_range ? st : nullptr;
+  };
+  const bool tiled = whole && ieq::tiled_stage_ok(p, ops, (int)sizeof(R));
+  const bool node = !(tiled && ieq::tiled_stage_pays(p, ops, (int)sizeof(R)));
+  auto is_2n = [&](int i) {  // names[i], names[i + 1] are the two halves of a 2N stage
+    if (i + 1 >= n || !node || !whole) return false;
+    const StageDesc *a = accepted(names[i]), *b = accepted(names[i + 1]);
+    return a && b && a->kind == K_STAGE && b->kind == K_2N && a->Y == b->out && a->out == b->P;
+  };
+  int pairs = 0;
+  for (int i = 0; i < n; ++i) pairs += is_2n(i);
+  void* copy = pairs >= 2 ? b1_copy_for(pr) : nullptr;
+  int fuse = copy ? pairs & ~1 : 0;  // stages to fuse: an even number
+  const bool used_copy = fuse > 0;
+  ieq::NodeTime<R> pend;  // set: time[1] is to become time[0] + add and has not been stored yet
+  auto take = [&](R* time) {
+    ieq::NodeTime<R> t = pend;
+    t.time = time;
+    pend = ieq::NodeTime<R>{};
+    return t;
+  };
+  auto flush = [&]() {
+    if (pend.set) ieq::gen_time<R>(s, pend.time, (double)pend.add, 1.0, 0);
+    pend = ieq::NodeTime<R>{};
+  };
+  int rc = IEQ_OK;
+  for (int i = 0; i < n && rc == IEQ_OK; ++i) {
+    if (!names[i]) {
+      rc = pr->fail(IEQ_ERR_ARGS, "NULL kernel name");
+      break;
+    }
+    const StageDesc* st = accepted(names[i]);
+    const int k0 = i;
+    auto F = [&](int k) { return (R*)A[k]; };
+    R* time = st ? (R*)A[st->nf + 3] : nullptr;
+    hipError_t e = hipSuccess;
+    if (st && st->kind == K_TIME) {
+      pend = ieq::NodeTime<R>{time, 1, (R)(st->tc * p.dt)};
+    } else if (st && st->kind == K_CALC_TIME) {
+      pend = ieq::NodeTime<R>{};  // calc_time sets both times
+      ieq::gen_time<R>(s, time, 0, p.dt, 1);
+    } else if (st && st->kind == K_CURL) {
+      const StageDesc* nx = i + 1 < n ? accepted(names[i + 1]) : nullptr;
+      const bool vel = nx && nx->kind == K_U;
+      e = ieq::node_pre<R>(p, ops, s, g, F(st->Y), F(st->nf), F(st->nf + 2), vel ? F(st->nf + 1) : nullptr,
+                           vel ? take(time) : ieq::NodeTime<R>{});
+      i += vel;
+    } else if (st && st->kind == K_U) {
+      e = ieq::node_pre<R>(p, ops, s, g, nullptr, nullptr, nullptr, F(st->nf + 1), take(time));
+    } else if (st && st->kind == K_STAGE && node) {
+      const bool two = fuse > 0 && is_2n(i);
+      const StageDesc* nx = two ? find_stage(names[i + 1]) : nullptr;
+      R* b1 = nullptr;
+      if (two) b1 = (R*)(A[0] == args[0] ? copy : args[0]);
+      e = ieq::node_stage<R>(p, ops, s, g, F(st->out), st->P >= 0 ? F(st->P) : nullptr, (R)st->cP, st->Q >= 0 ? F(st->Q) : nullptr,
+                             (R)st->cQ, F(st->Y), (R)(st->cD * p.dt), F(st->nf), F(st->nf + 1), take(time), b1,
+                             two ? (R)nx->cQ : R(0));
+      if (tiled) pr->tiled_used = true;
+      if (two) {
+        A[0] = b1;
+        if (nx->tc >= 0) pend = ieq::NodeTime<R>{time, 1, (R)nx->tc * (R)p.dt};
+        --fuse;
+        ++i;
+      }
+    } else {
+      flush();
+      rc = run_one<R>(pr, names[i], g, l, A.data(), nargs);
+      if (rc) break;
+    }
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e != hipSuccess) rc = hip_fail(pr, e, names[k0]);
+  }
+  flush();
+  if (used_copy) {
+    if (A[0] != args[0])  // only after an error between two stages
+      (void)hipMemcpyAsync(args[0], A[0], (size_t)3 * pr->info.stride * sizeof(R), hipMemcpyDeviceToDevice, s);
+    (void)hipEventRecord(pr->b1_copy_done, s);
+  }
+  return rc;
+}
+
 int run_list(ieq_program* pr, const char* const* names, int n, const uint32_t g[3], const uint32_t l[3], void* const* args,
              int nargs) {
-  for (int i = 0; i < n; ++i) {
-    if (!names[i]) return pr->fail(IEQ_ERR_ARGS, "NULL kernel name");
-    int rc = pr->info.real_bytes == 8 ? run_one<double>(pr, names[i], g, l, args, nargs)
-                                      : run_one<float>(pr, names[i], g, l, args, nargs);
-    if (rc) return rc;
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(pr, e, names[i]);
-  }
-  return IEQ_OK;
+  return pr->info.real_bytes == 8 ? run_list_t<double>(pr, names, n, g, l, args, nargs)
+                                  : run_list_t<float>(pr, names, n, g, l, args, nargs);
 }
 
 // Kernel time of one ABI call (hip events on the program's stream); destroys its events on
@@ -598,6 +729,8 @@ void ieq_program_release(ieq_program* prog) {
   ieq::fused_release(prog->fused);
   ieq::cg_release(prog->cg);
   if (prog->diag) (void)hipFree(prog->diag);
+  if (prog->b1_copy) (void)hipFree(prog->b1_copy);
+  if (prog->b1_copy_done) (void)hipEventDestroy(prog->b1_copy_done);
   delete prog;
 }
 
@@ -753,11 +886,13 @@ static int step_impl(ieq_program* prog, const char* integrator, long long nsteps
   }
   prog->tiled_used = false;
   if (rc == IEQ_OK && !used_fused) {
-    std::vector<const char*> names;
-    for (auto& s : sched) names.push_back(s.c_str());
+    std::vector<const char*> names;  // two steps at a time: an even number of 2N stages
+    for (int k = 0; k < 2; ++k)
+      for (auto& s : sched) names.push_back(s.c_str());
     uint32_t g[3] = {(uint32_t)prog->info.nx, (uint32_t)prog->info.ny, (uint32_t)prog->info.nz};
     uint32_t l[3] = {(uint32_t)prog->info.w_size, 1, 1};
-    for (long long k = 0; k < nsteps && rc == IEQ_OK; ++k) rc = run_list(prog, names.data(), (int)names.size(), g, l, args, nargs);
+    for (long long k = 0; k < nsteps && rc == IEQ_OK; k += 2)
+      rc = run_list(prog, names.data(), (int)(k + 1 < nsteps ? names.size() : sched.size()), g, l, args, nargs);
   }
   prog->last_path = rc == IEQ_OK ? (used_fused ? 1 : prog->tiled_used ? 2 : 0) : -1;
   tm.end(prog, rc, kernel_seconds);

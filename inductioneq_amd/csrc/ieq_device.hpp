@@ -145,6 +145,10 @@ __device__ inline void node_xyz(const Params& p, uint32_t ix, uint32_t iy, uint3
   z = (R)p.zmin + (R)iz * (R)p.dz;
 }
 
+// Sine and cosine of one argument (one range reduction for both).
+__device__ inline void sin_cos(double a, double& s, double& c) { sincos(a, &s, &c); }
+__device__ inline void sin_cos(float a, float& s, float& c) { sincosf(a, &s, &c); }
+
 // (st, ct) = (sin t, cos t): a caller that evaluates many nodes at one time forms them once.
 template <typename R>
 __device__ V3<R> b_analytical(const Params& p, uint32_t ix, uint32_t iy, uint32_t iz, R t, R st, R ct) {
@@ -182,10 +186,11 @@ __device__ V3<R> b_analytical(const Params& p, uint32_t ix, uint32_t iy, uint32_
     case TC_HALL_PERIODIC: {  // hall_periodic.h:15-34
       const R n1 = R(0.5773502691896258), al = R(0.5);
       R kk = (R(1) - al * al) / al;
-      R u1 = cos(kk * y + al * kk * t * n1) + sin(kk * z + al * kk * t * n1);
-      R u2 = cos(kk * z + al * kk * t * n1) + sin(kk * x + al * kk * t * n1);
-      R u3 = cos(kk * x + al * kk * t * n1) + sin(kk * y + al * kk * t * n1);
-      return {al * u1 + n1, al * u2 + n1, al * u3 + n1};
+      R sx, cx, sy, cy, sz, cz;
+      sin_cos(kk * x + al * kk * t * n1, sx, cx);
+      sin_cos(kk * y + al * kk * t * n1, sy, cy);
+      sin_cos(kk * z + al * kk * t * n1, sz, cz);
+      return {al * (cy + sz) + n1, al * (cz + sx) + n1, al * (cx + sy) + n1};
     }
     case TC_HALL_TRAVELLING_WAVE: {  // hall_travelling_wave.h:15-30
       const R uz = R(0.1);
@@ -211,7 +216,9 @@ __device__ V3<R> b_analytical(const Params& p, uint32_t ix, uint32_t iy, uint32_
 }
 
 template <typename R> __device__ V3<R> b_analytical(const Params& p, uint32_t ix, uint32_t iy, uint32_t iz, R t) {
-  return b_analytical<R>(p, ix, iy, iz, t, sin(t), cos(t));
+  R s, c;
+  sin_cos(t, s, c);
+  return b_analytical<R>(p, ix, iy, iz, t, s, c);
 }
 
 template <typename R> __device__ V3<R> b_boundary(const Params& p, uint32_t ix, uint32_t iy, uint32_t iz, R t) {
@@ -234,9 +241,11 @@ template <typename R> __device__ V3<R> u_analytical(const Params& p, uint32_t ix
     case TC_HALL_PERIODIC: {  // hall_periodic.h:75-91
       const R n1 = R(0.5773502691896258), al = R(0.5);
       R kk = (R(1) - al * al) / al;
-      return {cos(kk * y + al * kk * t * n1) + sin(kk * z + al * kk * t * n1),
-              cos(kk * z + al * kk * t * n1) + sin(kk * x + al * kk * t * n1),
-              cos(kk * x + al * kk * t * n1) + sin(kk * y + al * kk * t * n1)};
+      R sx, cx, sy, cy, sz, cz;
+      sin_cos(kk * x + al * kk * t * n1, sx, cx);
+      sin_cos(kk * y + al * kk * t * n1, sy, cy);
+      sin_cos(kk * z + al * kk * t * n1, sz, cz);
+      return {cy + sz, cz + sx, cx + sy};
     }
     case TC_HALL_TRAVELLING_WAVE: {  // hall_travelling_wave.h:141-157
       const R uz = R(0.1);

@@ -106,3 +106,72 @@ def test_tiled_stage_on_small_grids(ops, diss, real):
     prog, db, hb, path = _run_both(cfg, "SSPRK33", env={"IEQ_TILED_ZC": "4"})
     assert path == "tiled"
     _check(cfg, prog, db, hb, "SSPRK33", "%s %s" % (ops, diss))
+
+
+@pytest.mark.parametrize("integrator", ["SSPRK33", "SSPRK104", "KennedyCarpenterLewis2R54C", "CalvoFrancoRandez2R64",
+                                        "CarpenterKennedy2N54", "ToulorgeDesmet2N84F"])
+@pytest.mark.parametrize("per,hall,real", [(False, True, "double"), (True, True, "float"), (False, False, "double")])
+def test_kernel_list_equals_its_kernels_one_by_one(integrator, per, hall, real):
+    """A list shares launches (curl + velocity, time kernels, the halves of a 2N stage with a second copy of b1);
+    after it every argument is what the kernels leave one by one.  Whole lists of one and three steps (odd and even
+    numbers of 2N stages), and lists that end within a step: after a time kernel, between the halves of a stage.
+    The arithmetic per node is the same; 1e-13 (FP32 1e-6) of the largest value allows for other contractions."""
+    import torch
+
+    from inductioneq_amd.program import Program
+    from inductioneq_amd.schedules import rk_schedule
+    from test_gpu_tiled import _aos
+
+    cfg, B, U = _stage_case("4thOrder", (21, 10, 12), per, hall, None, real)
+    prog = Program(cfg)
+    names, nf = rk_schedule(integrator, hall, True)
+    rng = np.random.default_rng(8)
+    host = [_aos(cfg, B + 0.1 * rng.standard_normal(B.shape)) for _ in range(nf)]
+
+    def fresh():
+        a = [prog.upload_real4(h) for h in host] + [prog.vector(), prog.upload_real4(_aos(cfg, U)), prog.scalar(1.3)]
+        return a + [torch.tensor([0.2, 0.25], dtype=prog.torch_dtype, device="cuda")]
+
+    tol = 1e-13 if real == "double" else 1e-6
+    for lst in [names, names * 3] + [names[:k] for k in range(len(names) // 2, len(names) // 2 + 5)]:
+        one, all_ = fresh(), fresh()
+        for k in lst:
+            prog.run(k, one)
+        prog.run(lst, all_)
+        torch.cuda.synchronize()
+        for i, (x, y) in enumerate(zip(all_, one)):
+            x, y = (v[..., : cfg.num_nodes].double() if v.numel() > 2 else v.double() for v in (x, y))
+            assert float((x - y).abs().max()) <= tol * max(float(y.abs().max()), 1e-300), (len(lst), i)
+
+
+def test_lists_on_two_streams_share_the_second_copy_of_b1():
+    """Two solves of one program on two streams in turn, without a wait between the calls, equal the same solves
+    one after the other bit for bit."""
+    import torch
+
+    from inductioneq_amd.program import Program
+    from inductioneq_amd.schedules import rk_schedule
+    from test_gpu_tiled import _aos
+
+    cfg, B, U = _stage_case("6thOrder", (48, 40, 44), False, True, None, "double")
+    cfg.dt = 1e-5  # within the Hall term's stability limit: the states stay finite
+    prog = Program(cfg)
+    names, nf = rk_schedule("CarpenterKennedy2N54", True, True)
+
+    def solve(streams, scale):
+        regs = [[prog.upload_real4(_aos(cfg, B * c))] + [prog.vector() for _ in range(nf)] +
+                [prog.upload_real4(_aos(cfg, U)), prog.scalar(1.0), prog.time_buffer()] for c in scale]
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for s, a in zip(streams, regs):
+                with torch.cuda.stream(s):
+                    prog.use_current_stream()
+                    prog.run(names * 2, a)
+        torch.cuda.synchronize()
+        return [a[0].clone() for a in regs]
+
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    both = solve((s1, s2), (1.0, 0.5))
+    assert bool(torch.isfinite(both[0]).all())
+    assert torch.equal(both[0], solve((s1,), (1.0,))[0])
+    assert torch.equal(both[1], solve((s1,), (0.5,))[0])
