@@ -972,15 +972,17 @@ int clean_div_t(ieq_program* pr, R* b, R* phi, double thr, double rel, int max_i
   const double* tab = ieq::host_lap_table(I.opset, I.laplace, &nbl, &wl);
   if (!tab) return pr->fail(IEQ_ERR_SETTINGS, "no -Laplacian table for this operator set");
   std::memset(res, 0, sizeof(*res));
+  int rc = ieq::cg_run_t<R>(p, I, tab, nbl, wl, pr->stream, &pr->cg, b, phi, thr, rel, max_it, res, pr->err);
+  if (rc < 0) return IEQ_ERR_HIP;
+  if (rc == 0) return IEQ_OK;
+  // reference kernel sequence with host-side scalars (clean_div_CG.m:31-86)
   const size_t sbytes = (size_t)I.stride * sizeof(R);
   ScopedDev buf;  // scalar work fields + reduction partials
   HIP_TRY(pr, hipMalloc(&buf.p, 4 * sbytes + (size_t)I.num_groups * sizeof(R) + 64));
   R* tmp = (R*)buf.p;
   R *r = tmp, *u = tmp + I.stride, *q = tmp + 2 * I.stride, *dv = tmp + 3 * I.stride, *part = tmp + 4 * I.stride;
-  int rc = ieq::cg_run_t<R>(p, I, tab, nbl, wl, pr->stream, &pr->cg, b, phi, thr, rel, max_it, 16, res, pr->err);
-  if (rc < 0) return IEQ_ERR_HIP;
   const uint32_t g_dc[3] = {(uint32_t)(p.nx - 2 * p.bnodes), (uint32_t)(p.ny - 2 * p.bnodes), (uint32_t)(p.nz - 2 * p.bnodes)};
-  if (rc == 1) {  // reference kernel sequence with host-side scalars (clean_div_CG.m:31-76)
+  {
     HIP_TRY(pr, hipMemsetAsync(tmp, 0, 3 * sbytes, pr->stream));
     HIP_TRY(pr, hipMemsetAsync(phi, 0, sbytes, pr->stream));
     R* coef = part + I.num_groups;  // 1-element coefficient buffer

@@ -39,6 +39,8 @@ struct CgState {
 namespace {
 
 constexpr int kBlk = 256;
+constexpr int kAhead = 6;              // iterations the host launches ahead of the device (one takes 10 us or more, the host 6 us to launch it)
+constexpr long long kNodeLap = 150000;  // interior nodes up to which the Laplacian runs with a thread per node
 constexpr int kLapRows = 32;  // table rows held in LDS by k_cg_lap (2 * NUM_BOUNDS + 1 of the Laplacian)
 
 // Deterministic block reduction of one double (wave64 shuffles, then LDS).
@@ -74,26 +76,35 @@ __device__ inline double sum_partials_all(const double* part, unsigned int n, do
   return v;
 }
 
-struct LapArgs {
+constexpr int kMaxHW = 7;
+template <typename R> struct LapArgs {
   int nx, ny, nz, off;  // grid and BNODES
   int zc;               // planes per block
-  int nbl, wl, hw;      // table rows per side, width, half-width
+  int nbl, wl;          // table rows per side, width
   const double* tab;    // (2nbl+1) x wl, device copy
   double idx2, idy2, idz2;
-  unsigned int nblocks;
+  R cz[2 * kMaxHW + 1];  // central row of the table / dz^2, as REAL, offsets -hw .. hw
 };
 
-// Minimum waves per SIMD the register allocation of a 1024-thread Laplacian tile must allow.  A
-// workgroup of 64 x 16 threads puts 4 waves on each SIMD, so it needs at least 4 (the
-// unconstrained FP64 kernel at half-width 4 takes 133 VGPRs, 3 waves per SIMD, and would not
-// launch).  With one plane of loads in flight the kernels up to half-width 5 fit without
-// spilling (half-width 4: FP64 120 VGPRs, 4 waves; FP32 74 VGPRs, 6 waves).
-#ifndef IEQ_LAP_WAVES64
-#define IEQ_LAP_WAVES64 4
-#endif
-#ifndef IEQ_LAP_WAVES32
-#define IEQ_LAP_WAVES32 6
-#endif
+// The iteration's rr from the previous update's partials (the initial residual's for iteration 0), the
+// stop test and beta = rr / old (clean_div_CG.m:45-48), the same in every block; false once stopped.  The
+// host follows `progress` (host memory): iteration + 1, negative once stopped.
+__device__ inline bool cg_direction(CgState* st, const double* rr_part, unsigned int n_rr, int iter, int* progress, double* red,
+                                    double& beta) {
+  const double rr = sum_partials_all(rr_part, n_rr, red);
+  const double old = st->rrs[(iter + 1) & 1];
+  const bool go = rr > st->tol2 && (st->rel2 <= 0.0 || rr > st->rel2 * st->rr0) && iter < st->max_it;
+  if (threadIdx.x == 0 && threadIdx.y == 0 && blockIdx.x == 0) {
+    st->rr = rr;
+    st->old = old;
+    st->it = iter;
+    if (go) st->rrs[iter & 1] = rr;
+    else st->done = 1;
+    __hip_atomic_store(progress, go ? iter + 1 : -(iter + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  beta = rr / old;
+  return go;
+}
 
 // Fused direction update and Laplacian on [off, n-off)^3:
 //   u' = beta u + r (beta = rr/old),  q = -Lap u',  partial u'.q
@@ -106,69 +117,65 @@ struct LapArgs {
 // they always target a valid node (coordinates clamped into the grid) and land in raw
 // (u, r) registers; the masking and beta u + r happen only when a plane is used, so no
 // load is waited for before it is needed.  The per-plane barrier orders LDS traffic only.
+// The halo cells are numbered along the halo and thread i loads cell i (y rows first, so a
+// wave reads whole rows), one (u, r) pair per thread and plane instead of one pair for an x
+// cell and one for a y cell that most threads do not have.
+// What bounds it is the sum of LDS reads, L1 accesses and FMAs of a plane, not its latency (tiles
+// from 64 x 4 to 64 x 16 measure the same), so the z row comes from scalar registers except on
+// boundary planes and the centre from the window: 16 LDS reads a node and plane instead of 27
+// (192^3 FP32, half-width 4: 37.8 -> 33.5 us; its four fields once take 23 us as a copy).  Stepping phi here, where
+// u is at hand, spares the update a field but costs more than it saves (192^3, an iteration: FP32 63.4 -> 67.0 us,
+// FP64 122.9 -> 134.3).  A second plane in flight gives nothing.
 // Tiles are handed out per XCD in contiguous ranges (x fastest, then y, then z-chunk), so
 // the halo rows of y-neighbours are read through one L2.
 template <typename R, int HW, int TY, int PD, int TX>
-__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY >= 1024 ? (sizeof(R) == 4 ? IEQ_LAP_WAVES32 : IEQ_LAP_WAVES64) : 1, 8))) void k_cg_lap(LapArgs a, const R* __restrict__ u, const R* __restrict__ r,
+__global__ __launch_bounds__(TX * TY) void k_cg_lap(LapArgs<R> a, const R* __restrict__ u, const R* __restrict__ r,
                                                     R* __restrict__ un, R* __restrict__ q, CgState* st,
-                                                    const double* rr_part, unsigned int n_rr, double* part, int iter) {
-  constexpr int LX = TX + 2 * HW, LY = TY + 2 * HW, Q = 2 * HW + 1;
-  __shared__ R s[2][LY][LX];
+                                                    const double* rr_part, unsigned int n_rr, double* part, int iter,
+                                                    int* progress) {
+  constexpr int LX = TX + 2 * HW, LY = TY + 2 * HW, Q = 2 * HW + 1, NT = TX * TY;
+  constexpr int NYH = 2 * HW * TX, NHALO = NYH + 2 * HW * TY, NH = (NHALO + NT - 1) / NT;  // halo cells, per thread
+  __shared__ R s[2][LY * LX];
   __shared__ double red[17];
   if (st->done) return;
-  // rr of this iteration from the previous update's partials (the initial residual's for
-  // iteration 0), the stop test, and beta = rr / old (clean_div_CG.m:45-48)
-  const double rr = sum_partials_all(rr_part, n_rr, red);
-  const double old = st->rrs[(iter + 1) & 1];
-  const bool go = rr > st->tol2 && (st->rel2 <= 0.0 || rr > st->rel2 * st->rr0) && iter < st->max_it;
-  if (threadIdx.x == 0 && threadIdx.y == 0 && blockIdx.x == 0) {
-    st->rr = rr;
-    st->old = old;
-    st->it = iter;
-    if (go) st->rrs[iter & 1] = rr;
-    else st->done = 1;
-  }
-  if (!go) return;
-  const R beta = (R)(rr / old);
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  double beta_d;
+  if (!cg_direction(st, rr_part, n_rr, iter, progress, red, beta_d)) return;
+  const R beta = (R)beta_d;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = tx + TX * ty;
   const int gx = a.nx - 2 * a.off, gy = a.ny - 2 * a.off, gz = a.nz - 2 * a.off;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int ntx = (gx + TX - 1) / TX, nty = (gy + TY - 1) / TY;
   const int bx = tile % ntx, by = (tile / ntx) % nty, bz = tile / (ntx * nty);
-  const int x = a.off + bx * TX + tx, y = a.off + by * TY + ty;
-  const int x0 = a.off + bx * TX, y0 = a.off + by * TY;
+  const int x0 = a.off + bx * TX, y0 = a.off + by * TY, x = x0 + tx, y = y0 + ty;
   const bool active = (x - a.off) < gx && (y - a.off) < gy;
   const unsigned RB = sizeof(R);
   const unsigned plb = (unsigned)(a.nx * a.ny) * RB;
   auto cl = [](int v, int n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); };
   auto inb = [](int v, int n) { return (unsigned)v < (unsigned)n; };
-  // In-plane byte offsets (clamped) and in-grid masks of the column and its halo cells.
-  // Every thread issues the same loads each plane: one x-halo cell (left or right; threads
-  // off the x edges load their own column again), one y-halo cell per NYH (below / above,
-  // or the own column), so the memory counter of a plane's loads is the same on every path.
-  constexpr int NYH = 2 * HW <= TY ? 1 : 2;
+  // In-plane byte offsets (clamped) and in-grid masks of the column and of this thread's halo cells; a
+  // thread without one re-reads a fixed node, so the memory counter is the same on every path.
   const unsigned oc = (unsigned)(cl(x, a.nx) + a.nx * cl(y, a.ny)) * RB;
   const bool colin = inb(x, a.nx) && inb(y, a.ny);
-  const bool hl = tx < HW, hr = tx >= TX - HW, hb = ty < HW, ht = ty >= TY - HW;
-  const int hxx = hl ? x0 - HW + tx : x + HW;  // x-halo cell (used when hl || hr)
-  const int hyb = y0 - HW + ty, hya = y + HW;    // y-halo cells below / above
-  const unsigned ohx = (hl || hr) ? (unsigned)(cl(hxx, a.nx) + a.nx * cl(y, a.ny)) * RB : oc;
-  unsigned ohy[NYH];
-  bool mhy[NYH];
-  if constexpr (NYH == 1) {
-    const int yy = hb ? hyb : hya;
-    ohy[0] = (hb || ht) ? (unsigned)(cl(x, a.nx) + a.nx * cl(yy, a.ny)) * RB : oc;
-    mhy[0] = inb(x, a.nx) && inb(yy, a.ny);
-  } else {
-    ohy[0] = hb ? (unsigned)(cl(x, a.nx) + a.nx * cl(hyb, a.ny)) * RB : oc;
-    ohy[1] = ht ? (unsigned)(cl(x, a.nx) + a.nx * cl(hya, a.ny)) * RB : oc;
-    mhy[0] = inb(x, a.nx) && inb(hyb, a.ny);
-    mhy[1] = inb(x, a.nx) && inb(hya, a.ny);
+  unsigned oh[NH];
+  int lh[NH];  // LDS index of the cell, -1: none
+  bool mh[NH];
+#pragma unroll
+  for (int k = 0; k < NH; ++k) {
+    const int h = tid + k * NT, hx = h - NYH;
+    int lx, ly;
+    if (h < NYH) {
+      const int row = h / TX;
+      lx = h % TX;
+      ly = row < HW ? row - HW : TY + row - HW;
+    } else {
+      const int col = hx % (2 * HW);
+      lx = col < HW ? col - HW : TX + col - HW;
+      ly = hx / (2 * HW);
+    }
+    lh[k] = h < NHALO ? (ly + HW) * LX + lx + HW : -1;
+    mh[k] = inb(x0 + lx, a.nx) && inb(y0 + ly, a.ny);
+    oh[k] = h < NHALO ? (unsigned)(cl(x0 + lx, a.nx) + a.nx * cl(y0 + ly, a.ny)) * RB : 0u;
   }
-  const bool mhx = inb(hxx, a.nx) && inb(y, a.ny);
-  // LDS destinations of the halo cells
-  const int lxc = hl ? tx : tx + 2 * HW;                   // x-halo column
-  const int lyb = ty, lya = ty + 2 * HW;                   // y-halo rows below / above
   // per-thread x/y rows
   R cx[Q], cy[Q];
   {
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
   __shared__ R sz[kLapRows][Q];
   {
     const int rows = 2 * a.nbl + 1, c0 = (a.wl - 1) / 2;
-    for (int i = ty * TX + tx; i < rows * Q; i += TX * TY) {
+    for (int i = tid; i < rows * Q; i += NT) {
       const int row = i / Q, k = i % Q, j = c0 - HW + k;
       sz[row][k] = (j >= 0 && j < a.wl) ? (R)(a.tab[row * a.wl + j] * a.idz2) : R(0);
     }
@@ -208,7 +215,6 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
   // with a load in flight is never copied (a copy would wait for the load).
   constexpr int NS = PD + 1;
   static_assert(NS >= 2 && NS <= 4, "1 <= PD <= 3");
-  constexpr int NH = 1 + NYH;      // halo cells per thread and plane: x, then y
   R w[Q];                          // u' of the column, planes z-HW .. z+HW
   R lu[NS], lr[NS];                // raw column values
   R hu[NS][NH], hrw[NS][NH];       // raw halo values
@@ -219,12 +225,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
   };
   auto load_halo = [&](R* uu, R* rr, int zz) {  // unconditional: every path issues 2*NH loads
     const unsigned pz = (unsigned)cl(zz, a.nz) * plb;
-    uu[0] = ldo(u, ohx + pz);
-    rr[0] = ldo(r, ohx + pz);
 #pragma unroll
-    for (int k = 0; k < NYH; ++k) {
-      uu[1 + k] = ldo(u, ohy[k] + pz);
-      rr[1 + k] = ldo(r, ohy[k] + pz);
+    for (int k = 0; k < NH; ++k) {
+      uu[k] = ldo(u, oh[k] + pz);
+      rr[k] = ldo(r, oh[k] + pz);
     }
   };
 #pragma unroll
@@ -245,15 +249,11 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
   auto body = [&](auto slot, int zi) {
     constexpr int S = decltype(slot)::value, SN = (S + PD) % NS;
     const int z = z0 + zi;
-    auto& sp = s[zi & 1];
-    sp[ty + HW][tx + HW] = w[HW];
-    if (hl || hr) sp[ty + HW][lxc] = dir(hu[S][0], hrw[S][0], mhx);
-    if constexpr (NYH == 1) {
-      if (hb || ht) sp[hb ? lyb : lya][tx + HW] = dir(hu[S][1], hrw[S][1], mhy[0]);
-    } else {
-      if (hb) sp[lyb][tx + HW] = dir(hu[S][1], hrw[S][1], mhy[0]);
-      if (ht) sp[lya][tx + HW] = dir(hu[S][2], hrw[S][2], mhy[1]);
-    }
+    R* sp = s[zi & 1];
+    sp[(ty + HW) * LX + tx + HW] = w[HW];
+#pragma unroll
+    for (int k = 0; k < NH; ++k)
+      if (lh[k] >= 0) sp[lh[k]] = dir(hu[S][k], hrw[S][k], mh[k]);
     // loads PD planes ahead (halo first), in flight across PD barriers and computes; past the
     // chunk they read a clamped plane and are never used
     load_halo(hu[SN], hrw[SN], z + PD);
@@ -261,9 +261,15 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
     lds_barrier();
     if (active && zi < zn) {
       const int rz = bound_row((uint32_t)z, (uint32_t)a.nz, a.nbl, 0);
-      R acc = R(0);
+      const R *sx = sp + (ty + HW) * LX + tx, *sy = sp + ty * LX + tx + HW;
+      auto apply = [&](auto zrow) {
+        R acc = R(0);
 #pragma unroll
-      for (int k = 0; k < Q; ++k) acc = acc + cx[k] * sp[ty + HW][tx + k] + cy[k] * sp[ty + k][tx + HW] + sz[rz][k] * w[k];
+        for (int k = 0; k < Q; ++k)
+          acc = acc + cx[k] * (k == HW ? w[HW] : sx[k]) + cy[k] * (k == HW ? w[HW] : sy[k * LX]) + zrow(k) * w[k];
+        return acc;
+      };
+      const R acc = rz == a.nbl ? apply([&](int k) { return a.cz[k]; }) : apply([&](int k) { return sz[rz][k]; });
       const unsigned o = oc + (unsigned)z * plb;
       sto(un, o, w[HW]);
       sto(q, o, acc);
@@ -284,6 +290,70 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(TX * TY
   }
   const double bs = block_sum(dot, red);
   if (tx == 0 && ty == 0) part[tile] = bs;
+}
+
+// The same with a thread per node, for grids with too few tiles to fill the chip: a block takes 64
+// consecutive nodes of an interior xy-plane, three of its waves the stencil along one direction each and
+// the fourth the node itself.  All loads are in flight while the partials are summed.  40^3 FP64,
+// half-width 4: 7.0 us, where the z-march takes 22 us in 15 workgroups.
+template <typename R, int HW>
+__global__ __launch_bounds__(256) void k_cg_lap_node(LapArgs<R> a, const R* __restrict__ u, const R* __restrict__ r, R* __restrict__ un,
+                                                     R* __restrict__ q, CgState* st, const double* rr_part, unsigned int n_rr,
+                                                     double* part, int iter, int* progress) {
+  constexpr int Q = 2 * HW + 1;
+  __shared__ double red[17];
+  __shared__ R tab[3][kLapRows * Q];
+  __shared__ R sum[3][64];
+  if (st->done) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int gx = a.nx - 2 * a.off, gxy = gx * (a.ny - 2 * a.off), segs = (gxy + 63) / 64;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), zt = tile / segs, jt = (tile - zt * segs) * 64 + lane, j = min(jt, gxy - 1);
+  const int i3[3] = {a.off + j % gx, a.off + j / gx, a.off + zt}, n3[3] = {a.nx, a.ny, a.nz};
+  const int nxy = a.nx * a.ny, st3[3] = {1, a.nx, nxy};
+  const unsigned o = (unsigned)(i3[0] + a.nx * i3[1] + nxy * i3[2]) * (unsigned)sizeof(R);
+  const int d = wave < 3 ? wave : 0, i = wave == 0 ? i3[0] : wave == 1 ? i3[1] : i3[2], n = n3[d];
+  R uu[Q], rr[Q];
+  if (wave < 3) {
+#pragma unroll
+    for (int k = -HW; k <= HW; ++k) {  // outside the grid: the node itself, with a zero below
+      const unsigned ok = o + (unsigned)((unsigned)(i + k) < (unsigned)n ? k * st3[d] : 0) * (unsigned)sizeof(R);
+      uu[k + HW] = ldo(u, ok);
+      rr[k + HW] = ldo(r, ok);
+    }
+    const double ih2 = d == 0 ? a.idx2 : d == 1 ? a.idy2 : a.idz2;
+    const int c0 = (a.wl - 1) / 2;
+    for (int e = lane; e < (2 * a.nbl + 1) * Q; e += 64) {
+      const int jc = c0 - HW + e % Q;
+      tab[d][e] = jc >= 0 && jc < a.wl ? (R)(a.tab[e / Q * a.wl + jc] * ih2) : R(0);
+    }
+  } else {
+    uu[HW] = ldo(u, o);
+    rr[HW] = ldo(r, o);
+  }
+  double beta_d;
+  if (!cg_direction(st, rr_part, n_rr, iter, progress, red, beta_d)) return;
+  const R beta = (R)beta_d;
+  if (wave < 3) {
+    const int row = bound_row((uint32_t)i, (uint32_t)n, a.nbl, 0);
+    R acc = R(0);
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+      const R v = (unsigned)(i + k - HW) < (unsigned)n ? beta * uu[k] + rr[k] : R(0);
+      acc = acc + tab[d][row * Q + k] * v;
+    }
+    sum[d][lane] = acc;
+  }
+  __syncthreads();
+  if (wave < 3) return;
+  const R w = beta * uu[HW] + rr[HW], acc = (sum[0][lane] + sum[1][lane]) + sum[2][lane];
+  double dot = 0.0;
+  if (jt < gxy) {
+    sto(un, o, w);
+    sto(q, o, acc);
+    dot = (double)w * (double)acc;
+  }
+  for (int k = 32; k > 0; k >>= 1) dot += __shfl_xor(dot, k, 64);
+  if (lane == 0) part[tile] = dot;
 }
 
 // One workgroup, after the last enqueued iteration when the stop test never held: rr of the
@@ -356,28 +426,20 @@ __global__ __launch_bounds__(256) void k_cg_init_state(const double* part, unsig
   }
 }
 
-#ifndef IEQ_LAP_PD
-#define IEQ_LAP_PD 1
-#endif
-constexpr int kLapPD = IEQ_LAP_PD;  // planes of the Laplacian's z-march in flight per thread
-#ifndef IEQ_LAP_TY
-#define IEQ_LAP_TY 16
-#endif
-#ifndef IEQ_LAP_TX
-#define IEQ_LAP_TX 64
-#endif
-// Shape of a Laplacian tile (TX x TY threads) for stencil half-width hw: 64 x 16 up to hw = 5;
-// the wider stencils hold more registers (they would spill at 4 waves per SIMD) and run 64 x 8.
-constexpr int lap_ty(int hw) { return hw <= 5 ? IEQ_LAP_TY : 8; }
-constexpr int lap_tx(int hw) { return hw <= 5 ? IEQ_LAP_TX : 64; }
+constexpr int kLapPD = 1;  // planes of the Laplacian's z-march in flight per thread
+// Shape of a Laplacian tile (TX x TY threads) for stencil half-width hw: 32 x 16 up to hw = 5 (half-width 4,
+// FP64 / FP32: 192^3 65.6 / 36.0 us, 128^3 and 96^3 22.7 / 15.2 us; 64 x 8 68.0 / 35.9 and 24.5 / 17.6 us; 64 x 16
+// spills), 64 x 8 for the wider stencils.
+constexpr int lap_ty(int hw) { return hw <= 5 ? 16 : 8; }
+constexpr int lap_tx(int hw) { return hw <= 5 ? 32 : 64; }
 
-template <typename R, int HW, int TY>
-void launch_lap(const LapArgs& a, const R* u, const R* r, R* un, R* q, CgState* st, const double* rr_part, unsigned int n_rr,
-                double* part, int iter, hipStream_t s) {
-  const int gx = a.nx - 2 * a.off, gy = a.ny - 2 * a.off, gz = a.nz - 2 * a.off;
-  constexpr int TX = lap_tx(HW);
-  const int grid = ((gx + TX - 1) / TX) * ((gy + TY - 1) / TY) * ((gz + a.zc - 1) / a.zc);
-  k_cg_lap<R, HW, TY, kLapPD, TX><<<grid, dim3(TX, TY), 0, s>>>(a, u, r, un, q, st, rr_part, n_rr, part, iter);
+// Launch of one iteration's Laplacian; zc = 0: a thread per node.
+template <typename R, int HW>
+void launch_lap(const LapArgs<R>& a, unsigned int blocks, const R* u, const R* r, R* un, R* q, CgState* st, const double* rr_part,
+                unsigned int n_rr, double* part, int iter, int* progress, hipStream_t s) {
+  constexpr int TX = lap_tx(HW), TY = lap_ty(HW);
+  if (a.zc == 0) k_cg_lap_node<R, HW><<<blocks, 256, 0, s>>>(a, u, r, un, q, st, rr_part, n_rr, part, iter, progress);
+  else k_cg_lap<R, HW, TY, kLapPD, TX><<<blocks, dim3(TX, TY), 0, s>>>(a, u, r, un, q, st, rr_part, n_rr, part, iter, progress);
 }
 
 // Planes per z-chunk: the smallest chunk whose grid fits in one round of resident
@@ -401,28 +463,42 @@ template <typename R, int HW, int TY> int lap_zc(int gx, int gy, int gz) {
 }  // namespace
 
 struct CgWork {
-  void* buf = nullptr;  // r, u, q (num_nodes each) + partials + state + table
+  void* buf = nullptr;  // r, u, q, u' (num_nodes each) + partials + state + table
   size_t bytes = 0;
+  struct Host {         // pinned
+    CgState st;
+    double norm2;
+    int progress;
+  }* host = nullptr;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 
 void cg_release(CgWork* w) {
   if (!w) return;
   if (w->buf) (void)hipFree(w->buf);
+  if (w->host) (void)hipHostFree(w->host);
+  if (w->e0) (void)hipEventDestroy(w->e0);
+  if (w->e1) (void)hipEventDestroy(w->e1);
   delete w;
 }
 
 template <typename R>
 int cg_run_t(const Params& p, const ieq_program_info& info, const double* host_tab, int nbl, int wl, hipStream_t s, CgWork** work,
-             R* b, R* phi, double abs_thr, double rel_tol, int max_it, int chunk, ieq_cg_result* res, std::string& err) {
+             R* b, R* phi, double abs_thr, double rel_tol, int max_it, ieq_cg_result* res, std::string& err) {
   const long long n = info.num_nodes;
   const int hw = (wl - 1) / 2;
-  if (hw < 1 || hw > 7 || info.periodic || 2 * nbl + 1 > kLapRows || !offsets_fit(p.nx, p.ny, p.nz, sizeof(R)))
+  if (hw < 1 || hw > kMaxHW || info.periodic || 2 * nbl + 1 > kLapRows || !offsets_fit(p.nx, p.ny, p.nz, sizeof(R)))
     return 1;  // not covered by the fused loop
-  const int TY = lap_ty(hw);
+  const int TX = lap_tx(hw), TY = lap_ty(hw);
   const int gx = p.nx - 2 * p.bnodes, gy = p.ny - 2 * p.bnodes, gz = p.nz - 2 * p.bnodes;
-  int zc = 8;
-  if (const char* e = getenv("IEQ_LAP_ZC")) zc = std::max(1, atoi(e));
-  else switch (hw) {
+  // A thread per node up to kNodeLap interior nodes, the z-march beyond, where its tiles fill more of the chip
+  // and it loads a node once instead of once per stencil point.  An iteration, node / z-march, FP32 and FP64:
+  // half-width 4: 40^3 11.6 / 18.6 and 12.4 / 21.9 us, 56^3 19.2 / 20.2 and 21.1 / 23.2, 64^3 24.0 / 21.3 and
+  // 27.3 / 24.2, 96^3 55.8 / 24.7 and 67.8 / 29.3; half-width 1: 40^3 10.4 / 14.1 and 10.7 / 16.1, 56^3
+  // 16.5 / 15.2 and 17.5 / 17.2.
+  int zc = 0;
+  if (const char* e = getenv("IEQ_LAP_ZC")) zc = std::max(0, atoi(e));
+  else if ((long long)gx * gy * gz > kNodeLap) switch (hw) {
     case 1: zc = lap_zc<R, 1, lap_ty(1)>(gx, gy, gz); break;
     case 2: zc = lap_zc<R, 2, lap_ty(2)>(gx, gy, gz); break;
     case 3: zc = lap_zc<R, 3, lap_ty(3)>(gx, gy, gz); break;
@@ -431,102 +507,120 @@ int cg_run_t(const Params& p, const ieq_program_info& info, const double* host_t
     case 6: zc = lap_zc<R, 6, lap_ty(6)>(gx, gy, gz); break;
     default: zc = lap_zc<R, 7, lap_ty(7)>(gx, gy, gz); break;
   }
-  const int TX = lap_tx(hw);
-  const unsigned int lap_blocks = (unsigned)(((gx + TX - 1) / TX) * ((gy + TY - 1) / TY) * ((gz + zc - 1) / zc));
-  const unsigned int vec_blocks = 1024;
+  const unsigned int lap_blocks = zc > 0 ? (unsigned)(((gx + TX - 1) / TX) * ((gy + TY - 1) / TY) * ((gz + zc - 1) / zc))
+                                         : (unsigned)((gx * gy + 63) / 64 * gz);
+  const unsigned int vec_blocks = (unsigned)std::min<long long>(1024, (n + kBlk - 1) / kBlk);
   const size_t fbytes = ((size_t)info.stride * sizeof(R) + 255) / 256 * 256;
-  const size_t part_bytes = (size_t)(lap_blocks + vec_blocks) * sizeof(double);  // u'.q partials, then r.r partials
+  // u'.q partials, then r.r partials (later the 1024 of the final divergence norm)
+  const size_t part_bytes = ((size_t)(lap_blocks + 1024) * sizeof(double) + 255) / 256 * 256;
   const size_t tab_bytes = (size_t)(2 * nbl + 1) * wl * sizeof(double);
-  const size_t need = 4 * fbytes + ((part_bytes + 255) / 256 * 256) + 256 + tab_bytes;
+  const size_t need = 4 * fbytes + part_bytes + 512 + tab_bytes;
   if (!*work) *work = new CgWork();
   CgWork* w = *work;
-  if (w->bytes < need) {
+  if (!w->host && hipHostMalloc(&w->host, sizeof(CgWork::Host)) != hipSuccess) return w->host = nullptr, err = "hipHostMalloc failed", -4;
+  if (!w->e0 && hipEventCreate(&w->e0) != hipSuccess) return w->e0 = nullptr, err = "event creation failed", -4;
+  if (!w->e1 && hipEventCreate(&w->e1) != hipSuccess) return w->e1 = nullptr, err = "event creation failed", -4;
+  const bool fresh = w->bytes < need;
+  if (fresh) {
     if (w->buf) (void)hipFree(w->buf);
     w->buf = nullptr;
     w->bytes = 0;
-    if (hipMalloc(&w->buf, need) != hipSuccess) return err = "hipMalloc failed", -4;
+    if (hipMalloc(&w->buf, need) != hipSuccess) return w->buf = nullptr, err = "hipMalloc failed", -4;
     w->bytes = need;
   }
   char* base = (char*)w->buf;
   R* r = (R*)base;
   R* ub[2] = {(R*)(base + fbytes), (R*)(base + 3 * fbytes)};  // direction registers, alternating
   R* q = (R*)(base + 2 * fbytes);
-  double* part_uq = (double*)(base + 4 * fbytes);
+  CgState* st = (CgState*)(base + 4 * fbytes);
+  double* norm2 = (double*)((char*)st + 256);
+  double* tab = (double*)((char*)st + 512);
+  double* part_uq = tab + (2 * nbl + 1) * wl;
   double* part_rr = part_uq + lap_blocks;
-  CgState* st = (CgState*)(base + 4 * fbytes + (part_bytes + 255) / 256 * 256);
-  double* tab = (double*)((char*)st + 256);
-  if (hipMemsetAsync(base, 0, 4 * fbytes, s) != hipSuccess || hipMemsetAsync(phi, 0, fbytes, s) != hipSuccess ||
-      hipMemsetAsync(st, 0, sizeof(CgState), s) != hipSuccess ||
-      hipMemcpyAsync(tab, host_tab, tab_bytes, hipMemcpyHostToDevice, s) != hipSuccess)
+  // The Laplacian writes interior nodes only, so u' and q stay 0 outside from call to call.  The first
+  // direction (u of iteration 0) and the result start from 0 everywhere, and so does r outside the interior
+  // (an alpha that is not finite has left a NaN there).
+  if ((fresh && (hipMemsetAsync(base, 0, 4 * fbytes, s) != hipSuccess ||
+                 hipMemcpyAsync(tab, host_tab, tab_bytes, hipMemcpyHostToDevice, s) != hipSuccess)) ||
+      hipMemsetAsync(r, 0, 2 * fbytes, s) != hipSuccess || hipMemsetAsync(phi, 0, (size_t)info.stride * sizeof(R), s) != hipSuccess ||
+      hipMemsetAsync(st, 0, sizeof(CgState), s) != hipSuccess)
     return err = "CG set-up failed", -4;
 
-  hipEvent_t e0, e1;
-  (void)hipEventCreate(&e0);
-  (void)hipEventCreate(&e1);
-  (void)hipEventRecord(e0, s);
+  (void)hipEventRecord(w->e0, s);
   // r = div B on the interior (calc_div_divcleaning, kernel_div_cleaning.cl:60-70)
-  const uint32_t g_dc[3] = {(uint32_t)(p.nx - 2 * p.bnodes), (uint32_t)(p.ny - 2 * p.bnodes), (uint32_t)(p.nz - 2 * p.bnodes)};
+  const uint32_t g_dc[3] = {(uint32_t)gx, (uint32_t)gy, (uint32_t)gz};
   gen_div<R>(p, info.opset, s, g_dc, b, r, p.bnodes);
   k_cg_init<R><<<vec_blocks, kBlk, 0, s>>>(r, n, part_rr);
   k_cg_init_state<<<1, 256, 0, s>>>(part_rr, vec_blocks, st, abs_thr * abs_thr, rel_tol * rel_tol, max_it);
 
-  LapArgs la;
+  LapArgs<R> la{};
   la.nx = p.nx;
   la.ny = p.ny;
   la.nz = p.nz;
   la.off = p.bnodes;
   la.nbl = nbl;
   la.wl = wl;
-  la.hw = hw;
   la.tab = tab;
   la.idx2 = 1.0 / (p.dx * p.dx);
   la.idy2 = 1.0 / (p.dy * p.dy);
   la.idz2 = 1.0 / (p.dz * p.dz);
-  la.nblocks = lap_blocks;
+  for (int k = 0; k <= 2 * hw; ++k) la.cz[k] = (R)(host_tab[nbl * wl + (wl - 1) / 2 - hw + k] * la.idz2);
   la.zc = zc;
-  CgState hst;
+  // The host stays kAhead iterations in front of the one the device has reached, so the device never waits for
+  // it and few launches are left over (they return at once) when the stop test holds.
+  volatile int* progress = &w->host->progress;
+  *progress = 0;
   int launched = 0;
-  while (launched < max_it) {
-    const int k = std::min(chunk, max_it - launched);
-    for (int i = 0; i < k; ++i) {
-      const int it = launched + i;
-      const R* u = ub[it & 1];
-      R* un = ub[(it + 1) & 1];
-      switch (hw) {
-        case 1: launch_lap<R, 1, lap_ty(1)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        case 2: launch_lap<R, 2, lap_ty(2)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        case 3: launch_lap<R, 3, lap_ty(3)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        case 4: launch_lap<R, 4, lap_ty(4)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        case 5: launch_lap<R, 5, lap_ty(5)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        case 6: launch_lap<R, 6, lap_ty(6)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-        default: launch_lap<R, 7, lap_ty(7)>(la, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, s); break;
-      }
-      k_cg_update<R><<<vec_blocks, kBlk, 0, s>>>(phi, un, r, q, n, st, part_uq, lap_blocks, part_rr, it);
+  while (launched < max_it && *progress >= 0) {
+    for (unsigned spin = 1; launched - *progress >= kAhead && *progress >= 0; ++spin) {
+      if (spin % 4096) continue;
+      const int before = *progress;
+      const hipError_t e = hipStreamQuery(s);
+      if (e == hipErrorNotReady) continue;
+      (void)hipGetLastError();
+      if (e != hipSuccess) return err = std::string("CG iteration: ") + hipGetErrorString(e), -4;
+      if (*progress == before) break;  // everything launched has ended without a further iteration: stopped at once
     }
-    launched += k;
-    if (hipMemcpyAsync(&hst, st, sizeof(CgState), hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
-      return err = "CG state read failed", -4;
-    if (hst.done) break;
+    if (launched - *progress >= kAhead) break;
+    const int it = launched++;
+    const R* u = ub[it & 1];
+    R* un = ub[(it + 1) & 1];
+    int* pr = &w->host->progress;
+    switch (hw) {
+      case 1: launch_lap<R, 1>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      case 2: launch_lap<R, 2>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      case 3: launch_lap<R, 3>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      case 4: launch_lap<R, 4>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      case 5: launch_lap<R, 5>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      case 6: launch_lap<R, 6>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+      default: launch_lap<R, 7>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
+    }
+    k_cg_update<R><<<vec_blocks, kBlk, 0, s>>>(phi, un, r, q, n, st, part_uq, lap_blocks, part_rr, it);
   }
   k_cg_finish<<<1, 256, 0, s>>>(part_rr, vec_blocks, st, launched);  // no-op once the stop test held
-  (void)hipEventRecord(e1, s);
-  (void)hipEventSynchronize(e1);
+  (void)hipEventRecord(w->e1, s);
+  // projection over the whole grid and the final divergence norm (clean_div_CG.m:78-86)
+  const uint32_t g_full[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz};
+  gen_proj<R>(p, info.opset, s, g_full, b, phi);
+  gen_div_norm2<R>(p, info.opset, s, b, part_rr, norm2);
+  if (hipMemcpyAsync(&w->host->st, st, sizeof(CgState), hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipMemcpyAsync(&w->host->norm2, norm2, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess)
+    return err = "CG kernel launch or state read failed", -4;
   float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, e0, e1);
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  if (hipGetLastError() != hipSuccess) return err = "CG kernel launch failed", -4;
-  if (hipMemcpy(&hst, st, sizeof(CgState), hipMemcpyDeviceToHost) != hipSuccess) return err = "CG state read failed", -4;
+  (void)hipEventElapsedTime(&ms, w->e0, w->e1);
+  const CgState& hst = w->host->st;
   res->iterations = hst.it;
   res->residual_norm = std::sqrt(hst.rr);
   res->divergence_norm_initial = std::sqrt(hst.rr0);
+  res->divergence_norm_final = std::sqrt(std::max(w->host->norm2, 0.0));
   res->seconds = ms * 1e-3;
   return 0;
 }
 
 template int cg_run_t<double>(const Params&, const ieq_program_info&, const double*, int, int, hipStream_t, CgWork**, double*,
-                              double*, double, double, int, int, ieq_cg_result*, std::string&);
+                              double*, double, double, int, ieq_cg_result*, std::string&);
 template int cg_run_t<float>(const Params&, const ieq_program_info&, const double*, int, int, hipStream_t, CgWork**, float*,
-                             float*, double, double, int, int, ieq_cg_result*, std::string&);
+                             float*, double, double, int, ieq_cg_result*, std::string&);
 
 }  // namespace ieq

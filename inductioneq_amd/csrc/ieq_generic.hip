@@ -2,49 +2,115 @@
 // (order/closure, periodic or bounded grid, flux forms, Hall, SATs, the three
 // dissipation variants, the -Laplacians).  These back every reference kernel name
 // accepted by ieq_run(); the fused kernels in ieq_fused.hip replace the hot ones.
+#include <algorithm>
+#include <type_traits>
+
 #include "ieq_device.hpp"
 #include "ieq_generic.hpp"
+#include "ieq_node.hpp"
+#include "ieq_stencil.hpp"
 
 namespace ieq {
 namespace {
 
 constexpr int BX = 64, BY = 4;
 
-// d/dx_d of a vector field (diff_x/y/z, SBP_operator.cl:12-51) or of its M-adjoint.
-template <typename R, int OPS, bool ADJ>
-__device__ inline V3<R> dvec(const Params& p, const R* f, uint32_t ix, uint32_t iy, uint32_t iz, int d) {
+// Derivatives of one component (diff_x/y/z, SBP_operator.cl:12-51) or their M-adjoints at the nodes of a
+// column (fixed x and y, the planes of a chunk): the rows and neighbour offsets along x and y are found
+// once per thread, those along z are uniform in a wave.  A wave with a node near an x (y) face takes its
+// general row there for all lanes.  One node per thread spends 300 instructions,
+// most of them on rows and indices: 192^3 FP32, 4th order, div B 66 -> 44 us, its norm 112 -> 33, projection 68 -> 41;
+// the four fields of div B once take 23 us as a copy.
+template <typename R, int OPS, bool ADJ> struct Column {
   using O = Op<OPS>;
-  constexpr int C = (O::W - 1) / 2;
-  const uint32_t n3[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz}, i3[3] = {ix, iy, iz};
-  int row = bound_row(i3[d], n3[d], O::NB, p.periodic);
-  V3<R> acc = zero3<R>();
-  for (int i = 0; i < O::W; ++i)
-    acc = acc + (R)(ADJ ? O::dadj(row, i) : O::d(row, i)) * ld3(f, p.stride, at_dir(p, ix, iy, iz, d, i - C));
-  R h = (R)hdir(p, d);
-  return mk(acc.x / h, acc.y / h, acc.z / h);
-}
+  static constexpr int W = O::W, C = (W - 1) / 2;
+  unsigned o;  // in-plane byte offset of the nodes
+  bool mx, my;
+  R cx[W], cy[W];
+  unsigned ox[W], oy[W];
+  __device__ static double coef(int row, int k) { return ADJ ? O::dadj(row, k) : O::d(row, k); }
+  __device__ __forceinline__ void init(const Params& p, int ix, int iy) {
+    const NodeAxis ax = node_axis<OPS>(ix, p.nx, p.periodic), ay = node_axis<OPS>(iy, p.ny, p.periodic);
+    const unsigned RB = sizeof(R);
+    o = (unsigned)(ix + p.nx * iy) * RB;
+    mx = __all(ax.mid);
+    my = __all(ay.mid);
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      cx[k] = (R)coef(mx ? O::NB : ax.row, k);
+      cy[k] = (R)coef(my ? O::NB : ay.row, k);
+      ox[k] = o + (unsigned)node_step(ax, k - C, p.periodic) * RB;
+      oy[k] = o + (unsigned)(node_step(ay, k - C, p.periodic) * p.nx) * RB;
+    }
+  }
+  // MX, MY, MZ: the central row is taken along x, y, z (compile-time, so that the loads of all directions of a
+  // node are one run without branches; with a branch per direction a plane waits for three load latencies).
+  // f: the component's plane iz.
+  template <bool MID> __device__ __forceinline__ R line(const Params& p, const R* f, const R (&c)[W], const unsigned (&off)[W], int d) const {
+    R acc = R(0);
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      const double m = coef(O::NB, k);  // a literal: zero entries of the central row drop out
+      if constexpr (MID) {
+        if (m != 0.0) acc = acc + (R)m * node_ld(f, off[k]);
+      } else {
+        acc = acc + c[k] * node_ld(f, off[k]);
+      }
+    }
+    return acc / (R)hdir(p, d);
+  }
+  template <bool MX> __device__ __forceinline__ R dx(const Params& p, const R* f) const { return line<MX>(p, f, cx, ox, 0); }
+  template <bool MY> __device__ __forceinline__ R dy(const Params& p, const R* f) const { return line<MY>(p, f, cy, oy, 1); }
+  // the central row without a wrap: fixed strides from the plane pointer
+  __device__ static __forceinline__ bool inner(const Params& p, int iz) {
+    constexpr int RR = O::ORDER / 2;
+    return iz >= RR && iz + RR < p.nz && (p.periodic || (iz >= O::NB && iz + O::NB < p.nz));
+  }
+  template <bool MZ> __device__ __forceinline__ R dz(const Params& p, const R* f, int iz) const {
+    const long long nxy = (long long)p.nx * p.ny;
+    R acc = R(0);
+    if constexpr (MZ) {
+#pragma unroll
+      for (int k = -C; k <= C; ++k) {
+        const double m = coef(O::NB, k + C);
+        if (m != 0.0) acc = acc + (R)m * node_ld(f + k * nxy, o);
+      }
+    } else {
+      const NodeAxis az = node_axis<OPS>(iz, p.nz, p.periodic);
+#pragma unroll
+      for (int k = -C; k <= C; ++k) acc = acc + (R)coef(az.row, k + C) * node_ld(f + node_step(az, k, p.periodic) * nxy, o);
+    }
+    return acc / (R)hdir(p, 2);
+  }
+  template <bool MX, bool MY, bool MZ> __device__ __forceinline__ R div(const Params& p, const R* b, int iz) const {
+    return dx<MX>(p, b) + dy<MY>(p, b + p.stride) + dz<MZ>(p, b + 2 * p.stride, iz);  // SBP_operator.cl:101-110
+  }
+  // body(mx, my, mz, iz) for the planes z0 .. z1 - 1 with the flags as compile-time constants
+  template <typename Body> __device__ __forceinline__ void planes(const Params& p, int z0, int z1, Body body) const {
+    using std::false_type;
+    using std::true_type;
+    auto march = [&](auto x, auto y) {
+      for (int iz = z0; iz < z1; ++iz) {
+        if (inner(p, iz)) body(x, y, true_type{}, iz);
+        else body(x, y, false_type{}, iz);
+      }
+    };
+    if (mx && my) march(true_type{}, true_type{});
+    else if (my) march(false_type{}, true_type{});
+    else march(false_type{}, false_type{});
+  }
+};
 
-template <typename R, int OPS, bool ADJ>
-__device__ inline R dscal(const Params& p, const R* f, uint32_t ix, uint32_t iy, uint32_t iz, int d) {
-  using O = Op<OPS>;
-  constexpr int C = (O::W - 1) / 2;
-  const uint32_t n3[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz}, i3[3] = {ix, iy, iz};
-  int row = bound_row(i3[d], n3[d], O::NB, p.periodic);
-  R acc = R(0);
-  for (int i = 0; i < O::W; ++i) acc = acc + (R)(ADJ ? O::dadj(row, i) : O::d(row, i)) * f[at_dir(p, ix, iy, iz, d, i - C)];
-  return acc / (R)hdir(p, d);
-}
-
-template <typename R, int OPS> __device__ inline V3<R> curl_node(const Params& p, const R* f, uint32_t ix, uint32_t iy, uint32_t iz) {
-  V3<R> dx = dvec<R, OPS, false>(p, f, ix, iy, iz, 0), dy = dvec<R, OPS, false>(p, f, ix, iy, iz, 1),
-        dz = dvec<R, OPS, false>(p, f, ix, iy, iz, 2);
-  return {dy.z - dz.y, dz.x - dx.z, dx.y - dy.x};  // SBP_operator.cl:126-135
-}
-
-template <typename R, int OPS> __device__ inline R div_node(const Params& p, const R* f, uint32_t ix, uint32_t iy, uint32_t iz) {
-  return dvec<R, OPS, false>(p, f, ix, iy, iz, 0).x + dvec<R, OPS, false>(p, f, ix, iy, iz, 1).y +
-         dvec<R, OPS, false>(p, f, ix, iy, iz, 2).z;  // SBP_operator.cl:101-110
-}
+// A block of the column kernels: 256 consecutive nodes of an xy-plane of the NDRange (full lanes whatever the
+// sizes) and `zc` planes, blocks in contiguous ranges per XCD.
+#define IEQ_COLUMN_PREAMBLE(OFF)                                                                              \
+  const int segs = (int)((g.x * g.y + 255) / 256), tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;   \
+  const uint32_t jt = (uint32_t)(tile - ch * segs) * 256 + threadIdx.x;                                       \
+  if (jt >= g.x * g.y) return;                                                                                \
+  const int ix = (int)(jt % g.x) + (OFF), iy = (int)(jt / g.x) + (OFF);                                       \
+  const int z0 = ch * zc + (OFF), z1 = min(z0 + zc, (int)g.z + (OFF));                                        \
+  const long long S = p.stride, nxy = (long long)p.nx * p.ny;                                                 \
+  (void)S; (void)nxy;
 
 #define IEQ_NODE_PREAMBLE(OFF)                                            \
   uint32_t ix = blockIdx.x * BX + threadIdx.x, iy = blockIdx.y * BY + threadIdx.y, iz = blockIdx.z; \
@@ -113,20 +179,77 @@ template <typename R> __global__ __launch_bounds__(BX* BY) void k_init(Params p,
   else st3(f, S, idx, b_analytical<R>(p, ix, iy, iz, time[0]));
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_div(Params p, Range g, const R* b, R* out, int off) {
-  IEQ_NODE_PREAMBLE(off)
-  out[idx] = div_node<R, OPS>(p, b, ix, iy, iz);
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_div(Params p, Range g, int zc, const R* b, R* out, int off) {
+  IEQ_COLUMN_PREAMBLE(off)
+  Column<R, OPS, false> c;
+  c.init(p, ix, iy);
+  c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
+    sto(out + iz * nxy, c.o, c.template div<x.value, y.value, z.value>(p, b + iz * nxy, iz));
+  });
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_curl(Params p, Range g, const R* b, R* out) {
-  IEQ_NODE_PREAMBLE(0)
-  st3(out, S, idx, curl_node<R, OPS>(p, b, ix, iy, iz));
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_curl(Params p, Range g, int zc, const R* b, R* out) {
+  IEQ_COLUMN_PREAMBLE(0)
+  Column<R, OPS, false> c;
+  c.init(p, ix, iy);
+  c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {  // SBP_operator.cl:126-135
+    const R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
+    R* f = out + iz * nxy;
+    sto(f, c.o, c.template dy<y.value>(p, bz) - c.template dz<z.value>(p, by, iz));
+    sto(f + S, c.o, c.template dz<z.value>(p, bx, iz) - c.template dx<x.value>(p, bz));
+    sto(f + 2 * S, c.o, c.template dx<x.value>(p, by) - c.template dy<y.value>(p, bx));
+  });
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_grad(Params p, Range g, const R* f, R* out) {
-  IEQ_NODE_PREAMBLE(0)
-  st3(out, S, idx, mk(dscal<R, OPS, false>(p, f, ix, iy, iz, 0), dscal<R, OPS, false>(p, f, ix, iy, iz, 1),
-                      dscal<R, OPS, false>(p, f, ix, iy, iz, 2)));
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_grad(Params p, Range g, int zc, const R* f, R* out) {
+  IEQ_COLUMN_PREAMBLE(0)
+  Column<R, OPS, false> c;
+  c.init(p, ix, iy);
+  c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
+    const R* fz = f + iz * nxy;
+    R* o = out + iz * nxy;
+    sto(o, c.o, c.template dx<x.value>(p, fz));
+    sto(o + S, c.o, c.template dy<y.value>(p, fz));
+    sto(o + 2 * S, c.o, c.template dz<z.value>(p, fz, iz));
+  });
+}
+
+// Partial sums of the squared SBP norm of div B (calc_div + norm2_S, kernel_operator.cl:98-155): the
+// divergence in REAL as calc_div stores it, weights, squares and sums in double.  One partial per block, at
+// most kNormBlocks of them: runs of a plane beyond that many are walked with a stride.
+constexpr int kNormBlocks = 1024;
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_div_norm(Params p, int segs, int zc, const R* b, double* part) {
+  using O = Op<OPS>;
+  const int nxy = p.nx * p.ny, tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;
+  const int z0 = ch * zc, z1 = min(z0 + zc, p.nz);
+  double acc = 0.0;
+  for (int j = (tile - ch * segs) * 256 + (int)threadIdx.x; j < nxy; j += segs * 256) {
+    const int ix = j % p.nx, iy = j / p.nx;
+    Column<R, OPS, false> c;
+    c.init(p, ix, iy);
+    const double fxy = (p.dx / O::minv(bound_row(ix, p.nx, O::NB, p.periodic))) * (p.dy / O::minv(bound_row(iy, p.ny, O::NB, p.periodic)));
+    c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
+      const double d = (double)c.template div<x.value, y.value, z.value>(p, b + (long long)iz * nxy, iz);
+      acc += fxy * (p.dz / O::minv(bound_row(iz, p.nz, O::NB, p.periodic))) * (d * d);
+    });
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  __shared__ double sm[4];
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) part[tile] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+}
+// out[0] = sum of n partials in a fixed order.
+__global__ __launch_bounds__(256) void k_sum(const double* part, int n, double* out) {
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) acc += part[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  __shared__ double sm[4];
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) out[0] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
 }
 
 // -Laplacian of kernel_div_cleaning.cl:11-56 on the range offset by BNODES.
@@ -155,13 +278,23 @@ template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_lap(P
 }
 
 // projector_divcleaning (kernel_div_cleaning.cl:96-109): B +/- grad(phi), .xyz only
-template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_proj(Params p, Range g, R* b, const R* phi) {
-  IEQ_NODE_PREAMBLE(0)
-  if (p.laplace == 2) {
-    for (int d = 0; d < 3; ++d) b[d * S + idx] = b[d * S + idx] - dscal<R, OPS, true>(p, phi, ix, iy, iz, d);
-  } else {
-    for (int d = 0; d < 3; ++d) b[d * S + idx] = b[d * S + idx] + dscal<R, OPS, false>(p, phi, ix, iy, iz, d);
-  }
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_proj(Params p, Range g, int zc, R* b, const R* phi) {
+  IEQ_COLUMN_PREAMBLE(0)
+  auto apply = [&](auto adj, R sgn) {
+    Column<R, OPS, decltype(adj)::value> c;
+    c.init(p, ix, iy);
+    c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
+      const R* f = phi + iz * nxy;
+      R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
+      const R vx = node_ld(bx, c.o), vy = node_ld(by, c.o), vz = node_ld(bz, c.o);
+      const R dx = c.template dx<x.value>(p, f), dy = c.template dy<y.value>(p, f), dz = c.template dz<z.value>(p, f, iz);
+      sto(bx, c.o, vx + sgn * dx);
+      sto(by, c.o, vy + sgn * dy);
+      sto(bz, c.o, vz + sgn * dz);
+    });
+  };
+  if (p.laplace == 2) apply(std::true_type{}, R(-1));
+  else apply(std::false_type{}, R(1));
 }
 
 // calc_axpy (x = a x + y) / calc_xpay (x = x + a y), kernel_CG.cl:8-30
@@ -239,6 +372,16 @@ template <typename R> __global__ void k_soa_to_aos(const R* soa, R* aos, long lo
   aos[4 * i + 3] = R(0);
 }
 
+// Planes per block and blocks of the column kernels: about 4096 blocks, so that the chip is full and a thread
+// still has a few planes to share its rows between.
+int column_zc(Range g) {
+  const long long runs = (long long)((g.x * g.y + 255) / 256) * g.z;
+  return (int)std::max(1LL, std::min(16LL, runs / 4096));
+}
+unsigned column_blocks(Range g) {
+  const int zc = column_zc(g);
+  return ((g.x * g.y + 255) / 256) * ((g.z + zc - 1) / zc);
+}
 dim3 grid_of(Range g) { return dim3((g.x + BX - 1) / BX, (g.y + BY - 1) / BY, g.z); }
 
 }  // namespace
@@ -284,17 +427,25 @@ template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32
 
 template <typename R> void gen_div(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out, int off) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_div<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, b, out, off)))
+  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_div<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out, off)))
+}
+
+template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s, const R* b, double* part, double* out) {
+  const long long runs = ((long long)p.nx * p.ny + 255) / 256;
+  const int segs = (int)std::min<long long>(runs, kNormBlocks), most = kNormBlocks / segs, zc = (p.nz + most - 1) / most;
+  const int nb = segs * ((p.nz + zc - 1) / zc);
+  IEQ_OPS_SWITCH(ops, (k_div_norm<R, OPS><<<nb, 256, 0, s>>>(p, segs, zc, b, part)))
+  k_sum<<<1, 256, 0, s>>>(part, nb, out);
 }
 
 template <typename R> void gen_curl(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_curl<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, b, out)))
+  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_curl<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out)))
 }
 
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_grad<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, f, out)))
+  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_grad<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), f, out)))
 }
 
 template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
@@ -304,7 +455,7 @@ template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, cons
 
 template <typename R> void gen_proj(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* b, const R* phi) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_proj<R, OPS><<<grid_of(r), dim3(BX, BY), 0, s>>>(p, r, b, phi)))
+  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_proj<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, phi)))
 }
 
 template <typename R> void gen_axpy(const Params& p, hipStream_t s, const uint32_t g[3], R* x, const R* y, const R* a, int xpay) {
@@ -332,6 +483,7 @@ template <typename R> void gen_soa_to_aos(hipStream_t s, const R* soa, R* aos, l
   template void gen_time<R>(hipStream_t, R*, double, double, int);                                                           \
   template void gen_init<R>(const Params&, hipStream_t, const uint32_t*, R*, int, const R*);                                 \
   template void gen_div<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*, int);                             \
+  template void gen_div_norm2<R>(const Params&, int, hipStream_t, const R*, double*, double*);                              \
   template void gen_curl<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                 \
   template void gen_grad<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                 \
   template void gen_lap<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                  \

@@ -175,3 +175,110 @@ def test_lists_on_two_streams_share_the_second_copy_of_b1():
     assert bool(torch.isfinite(both[0]).all())
     assert torch.equal(both[0], solve((s1,), (1.0,))[0])
     assert torch.equal(both[1], solve((s1,), (0.5,))[0])
+
+
+@pytest.mark.parametrize("ops,lap,n,zc,real", [
+    ("4thOrder", "WIDE_STENCIL_DIRICHLET", (40, 36, 30), "8", "double"),        # half-width 4: ragged tiles, last chunk of 4
+    ("2ndOrder", "NARROW_STENCIL_DIRICHLET", (67, 18, 13), "2", "double"),      # half-width 1: three tiles in x, one plane left
+    ("2ndOrder", "WIDE_STENCIL_DIRICHLET", (34, 34, 9), "16", "float"),         # half-width 2: one chunk longer than the grid
+    ("2ndOrderExtended", "WIDE_STENCIL_LNS", (26, 24, 28), "12", "double"),     # half-width 3, no boundary nodes left out
+    ("4thOrder", "WIDE_STENCIL_LNS", (33, 17, 28), "10", "float"),              # half-width 5
+    ("4thOrderExtended", "WIDE_STENCIL_DIRICHLET", (70, 30, 32), "8", "double"),  # half-width 6: 64 x 8 tiles
+])
+def test_cg_march_equals_oracle(ops, lap, n, zc, real, monkeypatch):
+    """The Laplacian's z-march on small grids (there a thread per node is the rule) against the oracle after
+    8 iterations: FP64 1e-10 of the largest value as for the other form; FP32 1e-4 (rounding of 2^-24 over
+    27 terms and 8 iterations, times the condition of the first ones, which is below 60)."""
+    import torch
+
+    from inductioneq_amd.harness import clean_div_cg
+    from test_gpu_cg import _setup
+
+    monkeypatch.setenv("IEQ_LAP_ZC", zc)
+    prog, orc, cfg, aos = _setup(ops, lap, n, real)
+    aos = aos.astype(np.float32).astype(np.float64)
+    hb = aos.copy()
+    want = clean_div_cg(orc.cfg, orc, hb, 1e-9, 8)
+    db = prog.upload_real4(aos.astype(cfg.dtype))
+    got = prog.clean_div_cg(db, abs_threshold=1e-9, max_iterations=8)
+    torch.cuda.synchronize()
+    tol = 1e-10 if real == "double" else 1e-4
+    assert got["iterations"] == want["iterations"] == 8
+    phi_w, phi_g = want["phi"][: cfg.num_nodes], prog.download_real(got["phi"])[: cfg.num_nodes]
+    assert np.abs(phi_g - phi_w).max() <= tol * np.abs(phi_w).max()
+    b_g = prog.download_real4(db)[: cfg.num_nodes, :3]
+    assert np.abs(b_g - hb[: cfg.num_nodes, :3]).max() <= tol * np.abs(hb[:, :3]).max()
+
+
+@pytest.mark.parametrize("zc", [None, "8"])
+def test_cg_calls_leave_nothing_behind(zc, monkeypatch):
+    """A solve after one of a field without divergence (no iteration, field unchanged), one of NaN and one that
+    was cut short equals the first solve of a program bit for bit."""
+    import torch
+    from test_gpu_cg import _setup
+
+    if zc:
+        monkeypatch.setenv("IEQ_LAP_ZC", zc)
+    prog, _, cfg, aos = _setup("4thOrder", "WIDE_STENCIL_DIRICHLET", (35, 33, 34), "double")
+    first = prog.upload_real4(aos)
+    r1 = prog.clean_div_cg(first, abs_threshold=1e-6, max_iterations=25)
+    zero = prog.vector()
+    r0 = prog.clean_div_cg(zero, abs_threshold=1e-6, max_iterations=25)
+    assert r0["iterations"] == 0 and not zero.any() and not r0["phi"].any()
+    bad = torch.full_like(first, float("nan"))
+    prog.clean_div_cg(bad, abs_threshold=1e-6, max_iterations=25)
+    inf = torch.zeros_like(first)
+    inf[0, cfg.num_nodes // 2] = float("inf")
+    prog.clean_div_cg(inf, abs_threshold=1e-6, max_iterations=25)
+    prog.clean_div_cg(prog.upload_real4(2.0 * aos), abs_threshold=1e-6, max_iterations=3)
+    again = prog.upload_real4(aos)
+    r2 = prog.clean_div_cg(again, abs_threshold=1e-6, max_iterations=25)
+    torch.cuda.synchronize()
+    assert r1["iterations"] == r2["iterations"] == 25
+    assert torch.equal(first, again) and torch.equal(r1["phi"], r2["phi"])
+    assert r1["divergence_norm_final"] == r2["divergence_norm_final"]
+
+
+@pytest.mark.parametrize("ops,n,per,real", [
+    ("4thOrder", (200, 160, 101), False, "float"),         # 125 runs of 256 nodes, z-chunks of 3, the last of 2
+    ("6thOrder", (16, 16, 9), False, "double"),            # one run exactly, boundary rows on most planes
+    ("2ndOrderExtended", (257, 5, 6), True, "double"),     # the last run of 5 nodes
+    ("6thOrderExtended", (19, 27, 33), True, "float"),     # 513 nodes: two runs and one node
+    ("2ndOrder", (2, 85, 3), False, "double"),
+    ("4thOrderExtended", (300, 130, 61), True, "double"),  # periodic, z-chunks of 2, the last of 1
+])
+@pytest.mark.parametrize("part", [False, True])
+def test_column_kernels_equal_oracle(ops, n, per, real, part):
+    """Divergence, curl, gradient and projection on the whole grid and on a part of it whose other nodes stay as
+    they were: FP64 1e-12 of the largest value (three sums of at most 11 products), FP32 2e-5."""
+    import torch
+    from pyoracle import Oracle
+
+    from inductioneq_amd.program import Program
+    from test_gpu_parity import _aos, _relerr, _scal
+
+    lo, hi = (0.0, 2 * np.pi) if per else (-1.0, 1.0)
+    cfg = ProgramConfig(real=real, opset=ops, nx=n[0], ny=n[1], nz=n[2], xmin=lo, xmax=hi, ymin=lo, ymax=hi, zmin=lo,
+                        zmax=hi, periodic=per, testcase="hall_periodic" if per else "rotation_2D", w_size=64,
+                        laplace="WIDE_STENCIL_LNS")
+    prog, orc = Program(cfg), Oracle(cfg)
+    g = tuple(max(1, v - 1 - k) for k, v in enumerate(n)) if part else n
+    rng = np.random.default_rng(5)
+    hb, hp = _aos(cfg, rng.standard_normal((cfg.num_nodes, 3))), _scal(cfg, rng.standard_normal(cfg.num_nodes))
+    db, dp = prog.upload_real4(hb), prog.upload_real(hp)
+    tol = 1e-12 if real == "double" else 2e-5
+    hs, ds = _scal(cfg, np.full(cfg.num_nodes, 3.0)), prog.scalar(3.0)
+    orc.run("calc_div", [hb, hs], g=g)
+    prog.run("calc_div", [db, ds], g=g)
+    assert _relerr(prog.download_real(ds)[: cfg.num_nodes], hs[: cfg.num_nodes]) <= tol
+    for name, ha, da in (("calc_curl", hb, db), ("calc_grad", hp, dp)):
+        hv = _aos(cfg, np.full((cfg.num_nodes, 3), 3.0))
+        dv = prog.upload_real4(hv)
+        orc.run(name, [ha, hv], g=g)
+        prog.run(name, [da, dv], g=g)
+        assert _relerr(prog.download_real4(dv)[: cfg.num_nodes, :3], hv[: cfg.num_nodes, :3]) <= tol, name
+    if not per:
+        orc.run("projector_divcleaning", [hb, hp], g=g)
+        prog.run("projector_divcleaning", [db, dp], g=g)
+        torch.cuda.synchronize()
+        assert _relerr(prog.download_real4(db)[: cfg.num_nodes, :3], hb[: cfg.num_nodes, :3]) <= tol
