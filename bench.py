@@ -93,7 +93,7 @@ def traffic_summary(fetch_csv, write_csv, copyf_csv, copyw_csv, copy_mib=512):
 
 
 def stored_traffic(name, real):
-    """Traffic per RK stage of REAL type `real` (the k_hall_stage dispatch, or k_emf + k_stage of the two-kernel
+    """Traffic per RK stage of REAL type `real` (the k_hall_stage dispatch, or the EMF and stage kernels of a two-kernel
     form) from a committed summary, or None."""
     path = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(path):
@@ -101,7 +101,7 @@ def stored_traffic(name, real):
     d = json.load(open(path))
     kern = {k: v for k, v in d["kernels"].items() if ("<%s," % real) in k}
     one = [v["bytes"] for k, v in kern.items() if k.startswith("k_hall_stage")]
-    total = sum(one) if one else sum(v["bytes"] for k, v in kern.items() if k.startswith(("k_emf", "k_stage")))
+    total = sum(one) if one else sum(v["bytes"] for k, v in kern.items() if k.startswith(("k_emf", "k_stage", "k_brick")))
     return {"bytes_per_stage": total, "source": "profiles/" + name} if total else None
 
 

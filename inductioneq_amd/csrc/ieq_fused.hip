@@ -232,17 +232,48 @@ template <typename R> void launch_k(const void* k, int code, const FArgs<R>& a, 
   void* kargs[1] = {(void*)&arg};
   (void)hipLaunchKernel(k, dim3(tile_grid(a, code)), dim3(shape_tx(code), shape_ty(code)), kargs, 0, s);
 }
-template <typename R> void emf(int rr, int code, const FArgs<R>& a, hipStream_t s) { launch_k(emf_kernel<R>(rr, code), code, a, s); }
-template <typename R> void stage(int rr, int code, const FArgs<R>& a, bool hall, bool hod, hipStream_t s) {
-  launch_k(stage_kernel<R>(rr, code, a, hall, hod), code, a, s);
-}
-
 int env_int(const char* k, int dflt) {
   const char* v = std::getenv(k);
   return v && *v ? std::atoi(v) : dflt;
 }
 
+template <typename R> void emf(int rr, int code, const FArgs<R>& a, hipStream_t s) {
+  if (code == kBrickShape) return brick_emf<R>(rr, a, s);
+  launch_k(emf_kernel<R>(rr, code), code, a, s);
+}
+template <typename R> void stage(int rr, int code, const FArgs<R>& a, bool hall, bool hod, hipStream_t s) {
+  if (code == kBrickShape) return brick_stage<R>(rr, a, hall, hod, s);
+  launch_k(stage_kernel<R>(rr, code, a, hall, hod), code, a, s);
+}
+
 }  // namespace
+
+// Nodes with the idle lanes of 32 x 8 tiles.
+static long long brick_nodes(int nx, int ny, int nz) { return (long long)((nx + 31) / 32 * 32) * ((ny + 7) / 8 * 8) * nz; }
+
+// The z-march reads a node of the differentiated fields once, a brick (2 RR + 2) / 2 times, so the march wins where bytes
+// count and the brick where the march's chain of planes does.  A stage with its EMF (2N and SSPRK33 stages), march /
+// brick, us: FP32 half-width 3: 96^3 27.8 / 20.1, 128^3 45.1 / 38.0, 160^3 76.7 / 80.2 (with convection); 2: 128^3 40.6 /
+// 33.6, 160^3 66.5 / 65.2, 192^3 125 / 132; 1: 160^3 60.6 / 52.2.  FP64 half-width 3: 96^3 42.2 / 35.7, 112^3 60.5 / 61.7 (with
+// convection); 2: 128^3 65.6 / 62.2, 160^3 140 / 140; 1: 160^3 154 / 117.  Without the Hall term: FP32 3: 96^3 16.2 /
+// 12.1, 160^3 44.0 / 41.8; FP64 3: 96^3 23.2 / 21.6, 112^3 32.4 / 33.2; 1: 192^3 157 / 144.
+bool brick_pays(int rr, int real_bytes, int nx, int ny, int nz) {
+  if (const char* e = std::getenv("IEQ_BRICK")) return std::atoi(e) != 0;
+  static const double most[2][3] = {{8e6, 4e6, 1.4e6}, {8e6, 5e6, 3e6}};  // [FP32][half-width - 1]
+  return (double)brick_nodes(nx, ny, nz) <= most[real_bytes == 4][rr - 1];
+}
+
+// The EMF and stage brick kernels instead of k_hall_stage, which needs no E in memory but chains the planes of
+// both.  One kernel / bricks, us a stage (2N; SSPRK33 gains about 2 us more): FP32 half-width 3: 48^3 15.7 / 10.4, 96^3
+// 28.5 / 20.8, 120^3 39.2 / 37.3, 128^3 39.3 / 39.8 (with convection 96^3 34.4 / 23.0, 128^3 49.7 / 43.2, 160^3 82.4 / 86.4); 2:
+// 48^3 12.1 / 9.4, 96^3 20.8 / 18.5, 112^3 28.2 / 27.6, 128^3 30.5 / 36.1; 1: 48^3 9.2 / 8.7, 96^3 15.9 / 16.7.  FP64 half-width 3:
+// 48^3 19.7 / 15.1, 88^3 36.9 / 31.4, 96^3 36.9 / 37.2, 104^3 46.2 / 49.5 (with convection 96^3 45.9 / 43.4, 104^3 57.0 / 59.5); 2:
+// 64^3 15.5 / 16.4; 1: 64^3 10.7 / 14.5.  On the smallest grids of half-width 2 the second launch costs what is won.
+static bool brick_beats_hall(int rr, int real_bytes, bool conv, int nx, int ny, int nz) {
+  const double n = (double)brick_nodes(nx, ny, nz);
+  if (rr == 3) return n <= (real_bytes == 4 ? (conv ? 3e6 : 1.9e6) : conv ? 1.2e6 : 0.9e6);
+  return rr == 2 && real_bytes == 4 && n >= 6e4 && n <= 1.5e6;
+}
 
 int hall_shape_for(long long nx, long long ny, long long nz, int real_bytes) {
   const int forced = env_int("IEQ_HALL_TILE", -1);
@@ -493,7 +524,9 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     if (w->scratch) (void)hipFree(w->scratch);
     w->scratch = nullptr;
     w->scratch_bytes = 0;
-    if (hipMalloc(&w->scratch, vbytes) != hipSuccess) return err = "hipMalloc failed", IEQ_ERR_HIP;
+    if (hipMalloc(&w->scratch, vbytes) != hipSuccess) return w->scratch = nullptr, err = "hipMalloc failed", IEQ_ERR_HIP;
+    // the kernels write nodes only, and the copy back to b1 takes what follows them along
+    if (hipMemsetAsync(w->scratch, 0, vbytes, s) != hipSuccess) return err = "memset failed", IEQ_ERR_HIP;
     w->scratch_bytes = vbytes;
   }
 
@@ -507,7 +540,13 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
   // 28.5 us per stage).  The z-chunk is set below from the stage kernel's occupancy.
   const bool f64 = sizeof(R) == 8;
   const int ty_env = env_int("IEQ_FUSED_TY", f64 || p.nx % 64 != 0 ? 32 : 8);  // tile shape code: 4, 8 or 32 (32 x 8)
-  const int ty = ty_env == 4 || ty_env == 32 ? ty_env : 8;
+  // IEQ_BRICK = 0 / 1 forces the march / the bricks; a forced chunk, tile or split belongs to the march.
+  bool forced = false;
+  for (const char* k : {"IEQ_FUSED_TY", "IEQ_FUSED_ZC", "IEQ_EMF_ZC", "IEQ_FUSED_SPLIT", "IEQ_HALL_TILE"}) forced = forced || getenv(k);
+  const bool moving = mn[0] != 0.0 || mn[1] != 0.0 || mn[2] != 0.0;
+  const bool brick = env_int("IEQ_BRICK", !forced && (p.hall ? brick_beats_hall(rr, sizeof(R), moving, p.nx, p.ny, p.nz)
+                                                             : brick_pays(rr, sizeof(R), p.nx, p.ny, p.nz)));
+  const int ty = brick ? kBrickShape : ty_env == 4 || ty_env == 32 ? ty_env : 8;
   a.S = info.stride;
   a.c = coef;
   const double h[3] = {p.dx, p.dy, p.dz};
@@ -528,7 +567,7 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
   R* b1 = F[0];
   R* b1alt = nf == 2 ? (R*)w->scratch : nullptr;
   a.zc = env_int("IEQ_FUSED_ZC", 0);
-  if (a.zc < 1) {  // one round of resident workgroups for the plan's first stage kernel
+  if (a.zc < 1 && !brick) {  // one round of resident workgroups for the plan's first stage kernel
     FArgs<R> t = a;
     t.zc = 1;
     for (const StageSpec& st : plan) {
@@ -549,14 +588,14 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     }
     a.zc = pick_zc<R>(rr, ty, t, p.hall, hod);
   }
-  // One kernel per Hall stage unless split on request or the 32-bit byte offsets of the staged
-  // halo (which include the component) would not fit.
-  // FP32 stages with convection run faster as the EMF kernel + stage kernel pair (96^3 SSPRK33:
-  // 28.5 against 35.2 us per stage; 128^3: equal), every other Hall stage as one kernel.
-  const int split = env_int("IEQ_FUSED_SPLIT", (!f64 && a.conv) ? 1 : 0);
-  const bool one_kernel = p.hall && split == 0 && (long long)3 * info.stride * sizeof(R) < (1LL << 32);
+  // One kernel per Hall stage unless bricks are faster, it is split on request, or the 32-bit byte offsets of the
+  // staged halo (which include the component) would not fit.  Beyond the bricks' range FP32 stages of half-width
+  // 3 with convection run as the march pair up to 5 M nodes (160^3 79 against 82 us, 192^3 146 against 127).
+  const bool pair = !f64 && a.conv && rr == 3 && (long long)p.nx * p.ny * p.nz <= 5000000;
+  const int split = env_int("IEQ_FUSED_SPLIT", pair ? 1 : 0);
+  const bool one_kernel = p.hall && split == 0 && !brick && (long long)3 * info.stride * sizeof(R) < (1LL << 32);
   int zc_emf = 0, zc_hall = 0;
-  if (p.hall && !one_kernel) {
+  if (p.hall && !one_kernel && !brick) {
     zc_emf = env_int("IEQ_EMF_ZC", 0);
     if (zc_emf < 1) zc_emf = pick_zc_emf<R>(rr, ty, a);
   }

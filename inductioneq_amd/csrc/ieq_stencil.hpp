@@ -222,9 +222,15 @@ inline int stage_mode(bool two_n, int P, int Q, int Y) {
 // Fused plan of one step (same arithmetic as the reference schedule, time kernels dropped).
 bool fused_plan(const std::string& I, int hall, std::vector<StageSpec>& v, int& nf);
 
-// Fused forward launches (RR in {1, 2, 3}; tile shape code 4: 64 x 4, 8: 64 x 8, 32: 32 x 8).
+// Fused forward launches (RR in {1, 2, 3}; tile shape code 4: 64 x 4, 8: 64 x 8, 32: 32 x 8, kBrickShape: the
+// bricks of ieq_brick.hpp).
+constexpr int kBrickShape = 1;
 template <typename R> void launch_emf(int rr, int ty, const FArgs<R>& a, hipStream_t s);
 template <typename R> void launch_stage(int rr, int ty, const FArgs<R>& a, bool hall, bool hod, hipStream_t s);
+// Whether the EMF and stage kernels run with a workgroup per brick of nodes rather than as z-marches.
+bool brick_pays(int rr, int real_bytes, int nx, int ny, int nz);
+template <typename R> void brick_emf(int rr, const FArgs<R>& a, hipStream_t s);
+template <typename R> void brick_stage(int rr, const FArgs<R>& a, bool hall, bool hod, hipStream_t s);
 // z-chunk that makes the stage kernel's tile grid one round of resident workgroups.
 template <typename R> int pick_zc(int rr, int ty, const FArgs<R>& a, bool hall, bool hod);
 template <typename R> int pick_zc_emf(int rr, int ty, const FArgs<R>& a);

@@ -1,0 +1,79 @@
+"""EMF and stage kernels with a workgroup per 32 x 8 x 2 brick (IEQ_BRICK = 1 forces them, 0 the z-marches)
+against the oracle and against the z-marches, at sizes where a brick ends: one node past it or short of it in
+each direction, and grids narrower than a brick with its halo."""
+import numpy as np
+import pytest
+
+from inductioneq_amd.problems import hall_dt, random_modes_field
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ops,n,integrator,hall,diss,u,source,real", [
+    ("6thOrder", (31, 11, 13), "CarpenterKennedy2N54", True, "HIGH_ORDER", (0.0, 0.0, 0.0), "CENTRAL", "double"),
+    ("6thOrder", (33, 16, 10), "SSPRK33", True, "HIGH_ORDER", (0.3, -0.2, 0.1), "ZERO", "float"),
+    ("6thOrder", (12, 41, 11), "SSPRK104", False, "HIGH_ORDER", (0.3, -0.2, 0.1), "CENTRAL", "double"),
+    ("6thOrder", (64, 10, 15), "KennedyCarpenterLewis2R54C", True, None, (0.3, 0.1, -0.2), "ZERO", "double"),
+    ("4thOrder", (65, 8, 9), "CarpenterKennedy2N54", True, None, (0.0, 0.0, 0.0), "CENTRAL", "float"),
+    ("4thOrder", (8, 9, 40), "SSPRK33", True, "HIGH_ORDER", (0.2, 0.2, -0.1), "CENTRAL", "double"),
+    ("4thOrder", (32, 24, 8), "SSPRK104", True, "HIGH_ORDER", (0.0, 0.0, 0.0), "CENTRAL", "double"),
+    ("2ndOrder", (37, 17, 5), "SSPRK33", False, None, (0.3, -0.2, 0.1), "ZERO", "double"),
+    ("2ndOrder", (6, 5, 33), "CarpenterKennedy2N54", True, "HIGH_ORDER", (0.1, 0.3, 0.2), "ZERO", "float"),
+])
+def test_brick_steps_equal_oracle(ops, n, integrator, hall, diss, u, source, real):
+    """Two steps within the tolerances of the other fused kernels (1e-12, 2e-5 of the largest value), and what
+    follows the nodes in b1 stays 0 (the 2N schemes end an odd number of stages in another buffer)."""
+    import torch
+    from test_gpu_fused import TOL, _device_args, _Env, _oracle_steps, _periodic_cfg, _relerr
+
+    from inductioneq_amd.program import Program
+
+    cfg = _periodic_cfg(n, real, ops, hall, diss, u, ho_factor=0.5, form_source=source)
+    B0 = random_modes_field(n, seed=4, kmax=2, amp=0.3)
+    cfg.dt = hall_dt(B0, (cfg.dx, cfg.dy, cfg.dz), 6, c_hall=0.8, cfl=0.3)
+    prog = Program(cfg)
+    args = _device_args(prog, B0, 2 if "2N" in integrator else 3, u, 1.25)
+    with _Env(IEQ_BRICK=1):
+        prog.step(integrator, 1, args)
+        prog.step(integrator, 1, args)
+        torch.cuda.synchronize()
+    assert prog.last_step_fused
+    hb, _ = _oracle_steps(cfg, B0, integrator, 2, u, 1.25)
+    e = _relerr(args[0][:, : cfg.num_nodes].double().cpu().numpy().T, hb[0][: cfg.num_nodes, :3].astype(np.float64))
+    assert e <= TOL[real], e
+    assert not args[0][:, cfg.num_nodes:].any()
+
+
+@pytest.mark.parametrize("ops,n,hall,source,real", [
+    ("6thOrder", (33, 15, 11), True, "ZERO", "double"),
+    ("6thOrder", (10, 26, 13), True, "CENTRAL", "float"),
+    ("4thOrder", (32, 9, 12), False, "ZERO", "double"),
+    ("2ndOrder", (34, 8, 7), True, "ZERO", "double"),
+])
+def test_brick_adjoint_equals_march(ops, n, hall, source, real):
+    """Final state and gradients of a solve with snapshots.  The same sums in the same order per node: 1e-13 and
+    1e-6 of the largest value (contractions of products may differ); parameter gradients, sums over the nodes
+    whose terms cancel, 1e-10 and 1e-4."""
+    import torch
+    from test_gpu_fused import _Env, _periodic_cfg
+
+    from inductioneq_amd.adjoint import AdjointSolver
+    from inductioneq_amd.program import Program
+
+    cfg = _periodic_cfg(n, real, ops, hall, "HIGH_ORDER", ho_factor=0.5, form_source=source)
+    B0 = random_modes_field(n, seed=4, kmax=2, amp=0.3)
+    cfg.dt = hall_dt(B0, (cfg.dx, cfg.dy, cfg.dz), 6, c_hall=1.3, cfl=0.3)
+    got = {}
+    for brick in (0, 1):
+        prog = Program(cfg)
+        b0 = prog.vector()
+        b0[:, : cfg.num_nodes] = torch.as_tensor(B0.T.copy(), dtype=prog.torch_dtype)
+        with _Env(IEQ_BRICK=brick):
+            solver = AdjointSolver(prog, 5, 2)
+            bT = solver.forward(b0, (0.3, -0.2, 0.1), 0.8)
+            got[brick] = [bT.double(), *(torch.as_tensor(v).double().cpu() for v in solver.backward(bT * 0.5 + 0.1 * b0))]
+    eps, eps_p = (1e-13, 1e-10) if real == "double" else (1e-6, 1e-4)
+    assert float((got[0][0] - got[1][0]).abs().max()) <= eps * float(got[0][0].abs().max())
+    assert float((got[0][1] - got[1][1]).abs().max()) <= 10 * eps * float(got[0][1].abs().max())
+    for a, b in zip(got[0][2:], got[1][2:]):
+        assert float((a - b).abs().max()) <= eps_p * max(float(a.abs().max()), 1e-3)
