@@ -463,8 +463,15 @@ template <typename R> constexpr int hall_pd() { return sizeof(R) == 8 ? IEQ_HALL
 #define IEQ_HALL_SKEW 0
 #endif
 
+// Waves per SIMD the single-grid kernel is compiled for.  FP64 holds two, except half-width 2 without convection in
+// the three-register forms, which fits three (4th order SSPRK33, HO dissipation: 128^3 51.2 -> 45.9 us a stage, 192^3
+// 168 -> 145); with the 2N update (48.8 -> 52.2) or convection (47.7 -> 65.9) a third wave spills.
+template <typename R, int RR, bool CONV, int MODE> constexpr int hall_waves() {
+  return sizeof(R) == 4 ? IEQ_HALL_WAVES32 : RR == 2 && !CONV && MODE >= 2 ? 3 : IEQ_HALL_WAVES;
+}
+
 template <typename R, int RR, int TX, int TY, bool HOD, bool CONV, int MODE>
-__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? IEQ_HALL_WAVES32 : IEQ_HALL_WAVES, 8))) void k_hall_stage(
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(hall_waves<R, RR, CONV, MODE>(), 8))) void k_hall_stage(
     FArgs<R> a) {
   __shared__ HallLds<R, RR, TX, TY, 1 + IEQ_HALL_SKEW> L;
   int x0, y0, z0;
