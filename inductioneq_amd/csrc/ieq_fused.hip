@@ -11,8 +11,8 @@
 //               w = sign * (central D_HO row convolved with itself)
 // With the Hall term a stage is one kernel, k_hall_stage (ieq_hall_tiles.hpp), which forms E
 // on its tile and halo itself; IEQ_FUSED_SPLIT=1 selects the two-kernel form instead (k_emf
-// writes E, k_stage reads B and E).  Without the Hall term a stage is one k_stage.  All
-// kernels march along z with register queues of the z-stencil and stage one xy-plane (plus
+// writes E, k_stage reads B and E).  Without the Hall term a stage is one k_stage.  On moderate
+// grids the brick kernels (ieq_brick.hpp) take their place.  The others march along z with register queues of the z-stencil and stage one xy-plane (plus
 // halo) at a time in LDS for the x/y stencils.
 #include <algorithm>
 #include <cmath>

@@ -1,6 +1,5 @@
-// Reference-schedule kernels: one work-item per node, every option of the program
-// (order/closure, periodic or bounded grid, flux forms, Hall, SATs, the three
-// dissipation variants, the -Laplacians).  These back every reference kernel name
+// Reference-schedule kernels other than the stages, curl B / rho and calc_u (ieq_node_stage.inc): SBP operators
+// down a column of planes, and one work-item per node for the rest.  These back the reference kernel names
 // accepted by ieq_run(); the fused kernels in ieq_fused.hip replace the hot ones.
 #include <algorithm>
 #include <type_traits>
