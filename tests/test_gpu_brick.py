@@ -77,3 +77,37 @@ def test_brick_adjoint_equals_march(ops, n, hall, source, real):
     assert float((got[0][1] - got[1][1]).abs().max()) <= 10 * eps * float(got[0][1].abs().max())
     for a, b in zip(got[0][2:], got[1][2:]):
         assert float((a - b).abs().max()) <= eps_p * max(float(a.abs().max()), 1e-3)
+
+
+@pytest.mark.parametrize("real", ["double", "float"])
+def test_uniformity_check_sees_every_node(real):
+    """One node of one coefficient that differs, or is NaN or infinite, takes a step off the fused path: the first
+    and last node, those at the ends of a thread's four and of a block's 1024, and one in between."""
+    import torch
+    from test_gpu_fused import _device_args, _periodic_cfg
+
+    from inductioneq_amd.program import Program
+
+    cfg = _periodic_cfg((20, 17, 13), real, "4thOrder", diss=None)  # 4420 nodes: five blocks, the last of 324
+    cfg.dt = 1e-4
+    prog = Program(cfg)
+    n = cfg.num_nodes
+    args = _device_args(prog, np.ones((n, 3)), 3, (0.2, 0.0, -0.1), 1.25)
+    u, rho = args[4], args[5]
+
+    def fused():
+        prog.step("SSPRK33", 1, args)
+        torch.cuda.synchronize()
+        return prog.last_step_fused
+
+    assert fused()
+    for c, f in enumerate((u[0], u[1], u[2], rho.view(-1))):
+        for k in (0, 255, 256, 1023, 1024, 2500, 4095, 4096, n - 1):
+            old = float(f[k])
+            for bad in (old + 0.5, float("nan")) + ((float("inf"),) if k == 2500 else ()):
+                f[k] = bad
+                assert not fused(), (c, k, bad)
+            f[k] = old
+            for a in args[:3]:
+                a.zero_()
+        assert fused()
