@@ -593,14 +593,22 @@ int cg_run_t(const Params& p, const ieq_program_info& info, const double* host_t
   volatile int* progress = &w->host->progress;
   *progress = 0;
   int launched = 0;
+  // Nothing of a call that fails is left in flight (the workspace is the program's) or in the last error.
+  auto failed = [&](hipError_t e) {
+    (void)hipStreamSynchronize(s);
+    (void)hipGetLastError();
+    return err = std::string("CG kernel launch or state read failed: ") + hipGetErrorString(e), -4;
+  };
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return failed(e);
   while (launched < max_it && *progress >= 0) {
     for (unsigned spin = 1; launched - *progress >= kAhead && *progress >= 0; ++spin) {
       if (spin % 4096) continue;
       const int before = *progress;
-      const hipError_t e = hipStreamQuery(s);
+      e = hipStreamQuery(s);
+      (void)hipGetLastError();  // of the query: every launch so far has been looked at
       if (e == hipErrorNotReady) continue;
-      (void)hipGetLastError();
-      if (e != hipSuccess) return err = std::string("CG iteration: ") + hipGetErrorString(e), -4;
+      if (e != hipSuccess) return failed(e);
       if (*progress == before) break;  // everything launched has ended without a further iteration: stopped at once
     }
     if (launched - *progress >= kAhead) break;
@@ -618,6 +626,7 @@ int cg_run_t(const Params& p, const ieq_program_info& info, const double* host_t
       default: launch_lap<R, 7>(la, lap_blocks, u, r, un, q, st, part_rr, vec_blocks, part_uq, it, pr, s); break;
     }
     k_cg_update<R><<<vec_blocks, kBlk, 0, s>>>(phi, un, r, q, n, st, part_uq, lap_blocks, part_rr, it);
+    if ((e = hipGetLastError()) != hipSuccess) return failed(e);
   }
   k_cg_finish<<<1, 256, 0, s>>>(part_rr, vec_blocks, st, launched);  // no-op once the stop test held
   (void)hipEventRecord(w->e1, s);
@@ -625,10 +634,11 @@ int cg_run_t(const Params& p, const ieq_program_info& info, const double* host_t
   const uint32_t g_full[3] = {(uint32_t)p.nx, (uint32_t)p.ny, (uint32_t)p.nz};
   gen_proj<R>(p, info.opset, s, g_full, b, phi);
   gen_div_norm2<R>(p, info.opset, s, b, part_rr, norm2);
-  if (hipMemcpyAsync(&w->host->st, st, sizeof(CgState), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipMemcpyAsync(&w->host->norm2, norm2, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess)
-    return err = "CG kernel launch or state read failed", -4;
+  if ((e = hipGetLastError()) != hipSuccess ||
+      (e = hipMemcpyAsync(&w->host->st, st, sizeof(CgState), hipMemcpyDeviceToHost, s)) != hipSuccess ||
+      (e = hipMemcpyAsync(&w->host->norm2, norm2, sizeof(double), hipMemcpyDeviceToHost, s)) != hipSuccess ||
+      (e = hipStreamSynchronize(s)) != hipSuccess)
+    return failed(e);
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, w->e0, w->e1);
   const CgState& hst = w->host->st;

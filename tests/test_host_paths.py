@@ -1,0 +1,29 @@
+"""Host code of the library around its launches (error paths, launch shapes, ordering), with a recording HIP runtime
+in place of the real one: no GPU, no kernel runs."""
+import pytest
+from hostrun import build_hip, hostrun
+
+
+@pytest.fixture(scope="module")
+def hip(tmp_path_factory):
+    return build_hip(tmp_path_factory.mktemp("hip"))
+
+
+@pytest.mark.parametrize("nth", [4, 5])
+@pytest.mark.parametrize("zc", [None, "8"])
+def test_refused_cg_launch_fails_the_call(hip, nth, zc):
+    """A Laplacian (the call's 4th launch) or an update (5th) that cannot be launched: an error, as for the launches
+    before and after the iterations, and no solution reported."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=20, ny=20, nz=20, laplace="WIDE_STENCIL_DIRICHLET")
+        b, phi = ctypes.create_string_buffer(3 * 8064 * 8), ctypes.create_string_buffer(8064 * 8)
+        call = lambda: lib.ieq_clean_div_cg(h, ctypes.addressof(b), ctypes.addressof(phi), 1e-9, 0.0, 20, ctypes.byref(_capi.CgResult()))
+        assert call() == 0
+        names = [l[1] for l in log("launch")]
+        assert "k_cg_lap" in names[3] and "k_cg_update" in names[4], names
+        for n in (%d, len(names), 1):
+            fail("hipLaunchKernel", n)
+            assert call() != 0, n
+            assert H.host_hip_last() == 0  # and nothing is left for the next call to trip over
+        assert call() == 0
+    """ % nth, **({"IEQ_LAP_ZC": zc} if zc else {}))
