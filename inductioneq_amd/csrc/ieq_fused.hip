@@ -498,8 +498,14 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     if (!w->uniform && hipHostMalloc(&w->uniform, sizeof(UniformState)) != hipSuccess)
       return w->uniform = nullptr, err = "hipHostMalloc failed", IEQ_ERR_HIP;
     if (!w->seen) {
-      if (hipMalloc(&w->seen, sizeof(*w->seen)) != hipSuccess) return w->seen = nullptr, err = "hipMalloc failed", IEQ_ERR_HIP;
-      if (hipMemsetAsync(w->seen, 0, sizeof(*w->seen), s) != hipSuccess) return err = "memset failed", IEQ_ERR_HIP;
+      unsigned long long* seen = nullptr;  // kept once it is zero: with any other value a field that varies passes as uniform
+      if (hipMalloc(&seen, sizeof(*seen)) != hipSuccess) return err = "hipMalloc failed", IEQ_ERR_HIP;
+      if (hipMemsetAsync(seen, 0, sizeof(*seen), s) != hipSuccess) {
+        (void)hipFree(seen);
+        (void)hipGetLastError();  // the check below looks at it
+        return err = "memset failed", IEQ_ERR_HIP;
+      }
+      w->seen = seen;
     }
     w->uniform->varies = 0;
     const int nblk = (int)std::min<long long>(1024, (info.num_nodes + 1023) / 1024);

@@ -27,3 +27,21 @@ def test_refused_cg_launch_fails_the_call(hip, nth, zc):
             assert H.host_hip_last() == 0  # and nothing is left for the next call to trip over
         assert call() == 0
     """ % nth, **({"IEQ_LAP_ZC": zc} if zc else {}))
+
+
+def test_uniformity_word_is_zeroed_after_a_failed_attempt(hip):
+    """ieq_step's check compares its number with a device word that starts at 0; a word whose zeroing failed would
+    let a field that varies pass as uniform, so the next call makes and zeroes another."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=12, nz=12, periodic=True, testcase="uniform_flow")
+        args = far(7)
+        step = lambda: lib.ieq_step(h, b"SSPRK33", 1, 0, (P * 7)(*args), 7, None)
+        fail("hipMemsetAsync")
+        assert step() != 0
+        word = log("malloc")[0]
+        assert word[2] == "8" and ["free", word[1]] in log("free")
+        H.host_hip_clear()
+        assert step() == 0, lib.ieq_last_error(h)
+        kinds = [(l[0], l[2] if l[0] != "launch" else l[1]) for l in log("malloc", "memset", "launch")]
+        assert kinds[0] == ("malloc", "8") and kinds[1] == ("memset", "8") and "k_uniform_check" in kinds[2][1], kinds
+    """)
