@@ -45,3 +45,25 @@ def test_uniformity_word_is_zeroed_after_a_failed_attempt(hip):
         kinds = [(l[0], l[2] if l[0] != "launch" else l[1]) for l in log("malloc", "memset", "launch")]
         assert kinds[0] == ("malloc", "8") and kinds[1] == ("memset", "8") and "k_uniform_check" in kinds[2][1], kinds
     """)
+
+
+@pytest.mark.parametrize("n", [(1024, 1024, 1024), (1030, 1021, 2100)])
+def test_stage_kernels_launch_on_grids_of_2_to_the_30_nodes(hip, n):
+    """A list of the stage kernels on more nodes than one launch of four threads a node can take: no launch is
+    refused, and the blocks of 64 nodes of each kernel are those of every plane."""
+    hostrun(hip, """
+        n = %r
+        h = build(real="float", opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], hall=True, testcase="hall_periodic")
+        names = ["calc_curlB_rho_2_3args", "calc_u_3_args", "SSPRK33_2b"]
+        for k in names + [names]:
+            H.host_hip_clear()
+            assert run(h, k, far(7), n) == 0, lib.ieq_last_error(h)
+            assert not log("refused")
+            blocks = {}
+            for l in log("launch"):
+                if "node" in l[1]:
+                    assert l[3:5] == ["1", "1"] and l[5] == "256"
+                    blocks[l[1]] = blocks.get(l[1], 0) + int(l[2])
+            assert blocks or k == "calc_u_3_args"
+            assert all(v == (n[0] * n[1] + 63) // 64 * n[2] for v in blocks.values()), blocks
+    """ % (n,))
