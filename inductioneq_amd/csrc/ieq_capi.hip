@@ -569,8 +569,9 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
   int fuse = copy ? pairs & ~1 : 0;  // stages to fuse: an even number
   const bool used_copy = fuse > 0;
   ieq::NodeTime<R> pend;  // set: time[1] is to become time[0] + add and has not been stored yet
+  ieq::NodeTime<R> given;  // what the last launch was to store
   auto take = [&](R* time) {
-    ieq::NodeTime<R> t = pend;
+    ieq::NodeTime<R> t = given = pend;
     t.time = time;
     pend = ieq::NodeTime<R>{};
     return t;
@@ -587,6 +588,7 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
     }
     const StageDesc* st = accepted(names[i]);
     const int k0 = i;
+    given = ieq::NodeTime<R>{};
     auto F = [&](int k) { return (R*)A[k]; };
     R* time = st ? (R*)A[st->nf + 3] : nullptr;
     hipError_t e = hipSuccess;
@@ -624,7 +626,11 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
       if (rc) break;
     }
     if (e == hipSuccess) e = hipGetLastError();
-    if (e != hipSuccess) rc = hip_fail(pr, e, names[k0]);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      rc = hip_fail(pr, e, names[k0]);
+      if (given.set) pend = given;  // the time kernel came before the one that was refused
+    }
   }
   flush();
   if (used_copy) {

@@ -426,7 +426,7 @@ template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32
 
 template <typename R> void gen_div(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out, int off) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_div<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out, off)))
+  IEQ_OPS_SWITCH(ops, (k_div<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out, off)))
 }
 
 template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s, const R* b, double* part, double* out) {
@@ -439,12 +439,12 @@ template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s
 
 template <typename R> void gen_curl(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_curl<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out)))
+  IEQ_OPS_SWITCH(ops, (k_curl<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out)))
 }
 
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_grad<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), f, out)))
+  IEQ_OPS_SWITCH(ops, (k_grad<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), f, out)))
 }
 
 template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
@@ -454,7 +454,7 @@ template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, cons
 
 template <typename R> void gen_proj(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* b, const R* phi) {
   Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, if (column_blocks(r)) (k_proj<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, phi)))
+  IEQ_OPS_SWITCH(ops, (k_proj<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, phi)))
 }
 
 template <typename R> void gen_axpy(const Params& p, hipStream_t s, const uint32_t g[3], R* x, const R* y, const R* a, int xpay) {

@@ -67,3 +67,24 @@ def test_stage_kernels_launch_on_grids_of_2_to_the_30_nodes(hip, n):
             assert blocks or k == "calc_u_3_args"
             assert all(v == (n[0] * n[1] + 63) // 64 * n[2] for v in blocks.values()), blocks
     """ % (n,))
+
+
+@pytest.mark.parametrize("g", [(0, 12, 12), (12, 0, 12), (12, 12, 0)])
+def test_empty_ndrange_is_refused(hip, g):
+    """Every kernel over nodes refuses an NDRange without work-items, and a stage time that a time kernel of the
+    list set before the refused kernel is stored all the same."""
+    hostrun(hip, """
+        g = %r
+        h = build(opset="4thOrder", nx=12, ny=12, nz=12, hall=True, testcase="hall_periodic", laplace="WIDE_STENCIL_LNS")
+        two, seven = far(2), far(7)
+        for name, args in [("calc_div", two), ("calc_curl", two), ("calc_grad", two), ("calc_div_divcleaning", two),
+                           ("calc_laplace_divcleaning", two), ("projector_divcleaning", two),
+                           ("calc_curlB_rho_1_3args", seven), ("calc_u_3_args", seven), ("SSPRK33_2b", seven)]:
+            H.host_hip_clear()
+            assert run(h, name, args, g) == _capi.IEQ_ERR_HIP, name
+            assert not log("launch") and H.host_hip_last() == 0, name
+        for name in ("calc_u_3_args", "SSPRK33_2b"):
+            H.host_hip_clear()
+            assert run(h, ["SSPRK33_2a", name], seven, g) == _capi.IEQ_ERR_HIP
+            assert ["k_time" in l[1] for l in log("launch")] == [True]
+    """ % (g,))
