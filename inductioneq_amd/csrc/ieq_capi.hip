@@ -614,7 +614,8 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
                              (R)st->cQ, F(st->Y), (R)(st->cD * p.dt), F(st->nf), F(st->nf + 1), take(time), b1,
                              two ? (R)nx->cQ : R(0));
       if (tiled) pr->tiled_used = true;
-      if (two) {
+      if (e == hipSuccess) e = hipGetLastError();
+      if (two && e == hipSuccess) {  // a refused launch has written nothing: b1 is still where it was
         A[0] = b1;
         if (nx->tc >= 0) pend = ieq::NodeTime<R>{time, 1, (R)nx->tc * (R)p.dt};
         --fuse;

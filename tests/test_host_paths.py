@@ -88,3 +88,23 @@ def test_empty_ndrange_is_refused(hip, g):
             assert run(h, ["SSPRK33_2a", name], seven, g) == _capi.IEQ_ERR_HIP
             assert ["k_time" in l[1] for l in log("launch")] == [True]
     """ % (g,))
+
+
+@pytest.mark.parametrize("nth,copied", [(1, False), (2, True), (3, False), (4, True)])
+def test_list_that_fails_at_a_fused_stage_leaves_the_last_b1(hip, nth, copied):
+    """A 2N list whose nth stage is refused: after an odd number of stages b1 lives in the second copy and is copied
+    back, after an even number it is in the caller's field and stays as it is."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=10, nz=9)
+        names, nf = rk_schedule("CarpenterKennedy2N54", False, False)
+        n = 3 * 1088
+        bufs = [ctypes.create_string_buffer(bytes([k + 1]) * (8 * n), 8 * n) for k in range(nf + 4)]
+        args = [ctypes.addressof(b) for b in bufs]
+        assert run(h, names * 2, args, (12, 10, 9)) == 0
+        stages = [k for k, l in enumerate(log("launch")) if "k_node_stage" in l[1]]
+        H.host_hip_clear()
+        fail("hipLaunchKernel", stages[%d - 1] + 1)
+        assert run(h, names * 2, args, (12, 10, 9)) == _capi.IEQ_ERR_HIP
+        back = [l for l in log("memcpy") if int(l[1], 16) == args[0]]
+        assert len(back) == %d, log()
+    """ % (nth, copied))
