@@ -635,8 +635,10 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
   }
   flush();
   if (used_copy) {
-    if (A[0] != args[0])  // only after an error between two stages
-      (void)hipMemcpyAsync(args[0], A[0], (size_t)3 * pr->info.stride * sizeof(R), hipMemcpyDeviceToDevice, s);
+    if (A[0] != args[0]) {  // only after an error between two stages; the kernels write nodes, and so does this
+      const size_t pitch = (size_t)pr->info.stride * sizeof(R);
+      (void)hipMemcpy2DAsync(args[0], pitch, A[0], pitch, (size_t)pr->info.num_nodes * sizeof(R), 3, hipMemcpyDeviceToDevice, s);
+    }
     (void)hipEventRecord(pr->b1_copy_done, s);
   }
   return rc;

@@ -136,6 +136,14 @@ hipError_t hipMemcpyAsync(void* d, const void* a, size_t n, hipMemcpyKind, hipSt
 }
 hipError_t hipMemcpy(void* d, const void* a, size_t n, hipMemcpyKind k) { return hipMemcpyAsync(d, a, n, k, nullptr); }
 
+hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* a, size_t ap, size_t w, size_t h, hipMemcpyKind, hipStream_t s) {
+  IEQ_MAY_FAIL("hipMemcpyAsync");
+  note("memcpy " + hex(d) + " " + hex(a) + " " + std::to_string(w * h) + " " + hex(s));
+  if (dp * h <= kReal && ap * h <= kReal)
+    for (size_t k = 0; k < h; ++k) std::memcpy((char*)d + k * dp, (const char*)a + k * ap, w);
+  return hipSuccess;
+}
+
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   *s = (hipStream_t)std::malloc(8);
   return hipSuccess;

@@ -108,3 +108,17 @@ def test_list_that_fails_at_a_fused_stage_leaves_the_last_b1(hip, nth, copied):
         back = [l for l in log("memcpy") if int(l[1], 16) == args[0]]
         assert len(back) == %d, log()
     """ % (nth, copied))
+
+
+def test_b1_copied_back_after_an_error_keeps_what_follows_its_nodes(hip):
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=10, nz=9)  # 1080 nodes, components 1088 apart
+        names, nf = rk_schedule("CarpenterKennedy2N54", False, False)
+        bufs = [(ctypes.c_double * (3 * 1088))(*([7.0] * (3 * 1088))) for k in range(nf + 4)]
+        args = [ctypes.addressof(b) for b in bufs]
+        fail("hipLaunchKernel", 2)
+        assert run(h, names * 2, args, (12, 10, 9)) == _capi.IEQ_ERR_HIP
+        assert any(v != 7.0 for v in bufs[0][:1080])  # the second copy's bytes: the test runtime computes nothing
+        for c in range(3):
+            assert bufs[0][c * 1088 + 1080 : (c + 1) * 1088] == [7.0] * 8, c
+    """)
