@@ -21,6 +21,7 @@
 #include "ieq_fused.hpp"
 #include "ieq_generic.hpp"
 #include "ieq_node_stage.hpp"
+#include "ieq_shared.hpp"
 #include "ieq_tiled.hpp"
 
 using ieq::Params;
@@ -182,11 +183,9 @@ struct ieq_program {
                        // sequence with whole-grid stages of a program the tiled kernel covers
   bool tiled_used = false;  // the current ieq_run / ieq_step launched such a stage
   double* diag = nullptr;  // ieq_diagnostics: 3 * kDiagBlocks partials + the 3 results
-  // second copy of b1 for 2N stages that update it in the stage kernel (neighbours still read the first),
-  // the stream whose launches used it last and their end
+  // second copy of b1 for 2N stages that update it in the stage kernel (neighbours still read the first)
   void* b1_copy = nullptr;
-  hipStream_t b1_copy_stream = nullptr;
-  hipEvent_t b1_copy_done = nullptr;
+  ieq::SharedUse shared;  // of b1_copy and the fused steps' register
 
   bool has(const char* m) const { return modules.count(m) != 0; }
   int fail(int code, const std::string& msg) {
@@ -512,29 +511,12 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
 // being captured (an allocation or a wait on another stream's event would end the capture, and a replay would
 // share the buffer with calls it is not ordered with).
 void* b1_copy_for(ieq_program* pr) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(pr->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
-  if (!pr->b1_copy_done && hipEventCreateWithFlags(&pr->b1_copy_done, hipEventDisableTiming) != hipSuccess) {
-    pr->b1_copy_done = nullptr;
+  if (ieq::SharedUse::capturing(pr->stream)) return nullptr;
+  if (!pr->b1_copy && hipMalloc(&pr->b1_copy, (size_t)3 * pr->info.stride * pr->info.real_bytes) != hipSuccess) {
+    pr->b1_copy = nullptr;
     (void)hipGetLastError();
-    return nullptr;
   }
-  if (!pr->b1_copy) {
-    const size_t bytes = (size_t)3 * pr->info.stride * pr->info.real_bytes;
-    if (hipMalloc(&pr->b1_copy, bytes) != hipSuccess) {
-      pr->b1_copy = nullptr;
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    pr->b1_copy_stream = pr->stream;
-  } else if (pr->b1_copy_stream != pr->stream) {
-    if (hipStreamWaitEvent(pr->stream, pr->b1_copy_done, 0) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    pr->b1_copy_stream = pr->stream;
-  }
-  return pr->b1_copy;
+  return pr->b1_copy && pr->shared.enter(pr->stream) ? pr->b1_copy : nullptr;
 }
 
 // Runs a kernel list.  Neighbouring kernels of the time integrators share a launch where every kernel of the
@@ -567,7 +549,6 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
   for (int i = 0; i < n; ++i) pairs += is_2n(i);
   void* copy = pairs >= 2 ? b1_copy_for(pr) : nullptr;
   int fuse = copy ? pairs & ~1 : 0;  // stages to fuse: an even number
-  const bool used_copy = fuse > 0;
   ieq::NodeTime<R> pend;  // set: time[1] is to become time[0] + add and has not been stored yet
   ieq::NodeTime<R> given;  // what the last launch was to store
   auto take = [&](R* time) {
@@ -634,12 +615,9 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
     }
   }
   flush();
-  if (used_copy) {
-    if (A[0] != args[0]) {  // only after an error between two stages; the kernels write nodes, and so does this
-      const size_t pitch = (size_t)pr->info.stride * sizeof(R);
-      (void)hipMemcpy2DAsync(args[0], pitch, A[0], pitch, (size_t)pr->info.num_nodes * sizeof(R), 3, hipMemcpyDeviceToDevice, s);
-    }
-    (void)hipEventRecord(pr->b1_copy_done, s);
+  if (copy && A[0] != args[0]) {  // only after an error between two stages; the kernels write nodes, and so does this
+    const size_t pitch = (size_t)pr->info.stride * sizeof(R);
+    (void)hipMemcpy2DAsync(args[0], pitch, A[0], pitch, (size_t)pr->info.num_nodes * sizeof(R), 3, hipMemcpyDeviceToDevice, s);
   }
   return rc;
 }
@@ -739,7 +717,6 @@ void ieq_program_release(ieq_program* prog) {
   ieq::cg_release(prog->cg);
   if (prog->diag) (void)hipFree(prog->diag);
   if (prog->b1_copy) (void)hipFree(prog->b1_copy);
-  if (prog->b1_copy_done) (void)hipEventDestroy(prog->b1_copy_done);
   delete prog;
 }
 
@@ -753,6 +730,7 @@ int ieq_program_get_info(const ieq_program* prog, ieq_program_info* info) {
 
 int ieq_set_stream(ieq_program* prog, void* hip_stream) {
   if (!prog) return IEQ_ERR_ARGS;
+  if (prog->stream != (hipStream_t)hip_stream) prog->shared.leave(prog->stream);
   prog->stream = (hipStream_t)hip_stream;
   return IEQ_OK;
 }
@@ -839,6 +817,7 @@ int ieq_run(ieq_program* prog, const char* const* names, int n, const uint32_t g
   // such a list over the whole grid takes the fused kernels when the program qualifies.
   if (fused_allowed() && full_grid(prog, g) && match_rk_list(prog, names, n, nargs, &integ, &k)) {
     ieq::FusedOpts opt;
+    opt.shared = &prog->shared;
     opt.final_curl = true;  // every argument ends as after the listed kernels
     rc = ieq::fused_step(prog->p, prog->info, prog->stream, &prog->fused, integ, k, 0, args, opt, &used, prog->err);
   }
@@ -889,6 +868,7 @@ static int step_impl(ieq_program* prog, const char* integrator, long long nsteps
   int used_fused = 0;
   if (fused_allowed()) {
     ieq::FusedOpts opt;
+    opt.shared = &prog->shared;
     opt.uniform = uniform;
     rc = ieq::fused_step(prog->p, prog->info, prog->stream, &prog->fused, integrator, nsteps, variable_u, args, opt,
                          &used_fused, prog->err);

@@ -26,6 +26,7 @@
 #include "ieq_generic.hpp"
 #include "ieq_hall.hpp"
 #include "ieq_node_stage.hpp"
+#include "ieq_shared.hpp"
 #include "ieq_stencil.hpp"
 
 namespace ieq {
@@ -529,6 +530,7 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     if (hipMemsetAsync(w->scratch, 0, vbytes, s) != hipSuccess) return err = "memset failed", IEQ_ERR_HIP;
     w->scratch_bytes = vbytes;
   }
+  if (nf == 2 && !SharedUse::capturing(s) && !opt.shared->enter(s)) return err = "event wait failed", IEQ_ERR_HIP;
 
   FArgs<R> a{};
   a.nx = p.nx;

@@ -12,6 +12,7 @@ namespace ieq {
 
 struct Params;
 struct FusedWork;
+struct SharedUse;
 
 // Kernel names of one time step of `integrator` (compute_numerical_solution_setup.m:140-371).
 // Returns 0, or -1 for an unknown integrator.
@@ -24,6 +25,7 @@ struct FusedOpts {
   // leave curlB_rho = curl B / rho of the last stage's input, as the reference schedule does
   // (otherwise it holds a work field)
   bool final_curl = false;
+  SharedUse* shared = nullptr;  // ordering of the program's buffers between streams
 };
 
 // Advance nsteps with the fused kernels when the program qualifies (periodic grid,

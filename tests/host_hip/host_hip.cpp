@@ -18,7 +18,7 @@ std::string g_log;
 std::map<const void*, std::string> g_names;           // host stub -> kernel
 std::map<std::string, std::pair<int, int>> g_fail;     // call -> (calls until it fails, error)
 hipError_t g_last = hipSuccess;
-int g_capturing = 0;
+hipStream_t g_capturing = (hipStream_t)-1;  // the stream that records a graph
 hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;
 struct {
   dim3 grid, block;
@@ -56,7 +56,7 @@ extern "C" {
 const char* host_hip_log() { return g_log.c_str(); }
 void host_hip_clear() { g_log.clear(); }
 void host_hip_fail(const char* fn, int nth, int code) { g_fail[fn] = {nth, code}; }  // the nth call from now on
-void host_hip_capture(int on) { g_capturing = on; }
+void host_hip_capture(void* s) { g_capturing = (hipStream_t)s; }
 int host_hip_last() { return (int)g_last; }
 
 void** __hipRegisterFatBinary(const void*) {
@@ -163,9 +163,9 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
   note("wait " + hex(s) + " " + hex(e));
   return hipSuccess;
 }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
   IEQ_MAY_FAIL("hipStreamIsCapturing");
-  *st = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  *st = g_capturing == s ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {

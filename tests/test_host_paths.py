@@ -122,3 +122,45 @@ def test_b1_copied_back_after_an_error_keeps_what_follows_its_nodes(hip):
         for c in range(3):
             assert bufs[0][c * 1088 + 1080 : (c + 1) * 1088] == [7.0] * 8, c
     """)
+
+
+@pytest.mark.parametrize("call", ["step", "list"])
+def test_program_buffers_are_handed_from_stream_to_stream(hip, call):
+    """2N stages keep a second b1 with the program (fused steps and lists alike).  Leaving a stream marks the end of
+    its use there, the next call that uses it on another stream waits for the mark before it launches, and nothing
+    is marked or waited for while the stream stays the same or is being captured."""
+    hostrun(hip, """
+        fused = %r == "step"
+        h = build(opset="4thOrder", nx=16, ny=12, nz=12, periodic=fused, testcase="uniform_flow")
+        names, nf = rk_schedule("CarpenterKennedy2N54", False, False)
+        u3 = (ctypes.c_double * 3)(0.1, 0.0, 0.2)
+        bufs = [ctypes.create_string_buffer(3 * 2304 * 8) for _ in range(6)]
+
+        def go(stream, shared=True):
+            H.host_hip_clear()
+            assert lib.ieq_set_stream(h, P(stream)) == 0
+            a = [ctypes.addressof(b) for b in bufs]
+            if not shared:
+                assert run(h, "CarpenterKennedy2N54_1a", a, (16, 12, 12)) == 0
+            elif fused:
+                assert lib.ieq_step_uniform(h, b"CarpenterKennedy2N54", 1, u3, 1.0, (P * 6)(*a), 6, None) == 0
+            else:
+                assert run(h, names, a, (16, 12, 12)) == 0
+            lines = [(l[0], l[1] if l[0] == "wait" else l[2]) for l in log("wait", "record")]
+            n = [l[0] for l in log("wait", "record", "launch")].index("launch")
+            assert n == len(lines), "marks and waits come before the launches"
+            return lines
+
+        A, B, C, D = 0x1000, 0x2000, 0x3000, 0x4000
+        assert go(A) == go(A) == []
+        assert go(B) == [("record", hex(A)), ("wait", hex(B))]
+        assert go(B) == []
+        assert go(C, shared=False) == [("record", hex(B))]
+        assert go(A) == [("wait", hex(A))]  # B's mark: C has not used the buffer
+        H.host_hip_capture(P(D))
+        assert go(D) == [("record", hex(A))]
+        H.host_hip_capture(P(-1))
+        assert go(D) == [("wait", hex(D))]
+        assert go(A) == [("record", hex(D)), ("wait", hex(A))]
+        assert go(A) == []
+    """ % call)
