@@ -512,9 +512,13 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
 // share the buffer with calls it is not ordered with).
 void* b1_copy_for(ieq_program* pr) {
   if (ieq::SharedUse::capturing(pr->stream)) return nullptr;
-  if (!pr->b1_copy && hipMalloc(&pr->b1_copy, (size_t)3 * pr->info.stride * pr->info.real_bytes) != hipSuccess) {
-    pr->b1_copy = nullptr;
-    (void)hipGetLastError();
+  if (!pr->b1_copy) {
+    // Relaxed: an allocation would end a capture that goes on elsewhere, which the list's launches leave alone.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (hipMalloc(&pr->b1_copy, (size_t)3 * pr->info.stride * pr->info.real_bytes) != hipSuccess) pr->b1_copy = nullptr;
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!pr->b1_copy) (void)hipGetLastError();
   }
   return pr->b1_copy && pr->shared.enter(pr->stream) ? pr->b1_copy : nullptr;
 }

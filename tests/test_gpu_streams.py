@@ -39,3 +39,43 @@ def test_fused_2n_steps_on_two_streams(ops, n, real):
     assert bool(torch.isfinite(both[0]).all())
     assert torch.equal(both[0], solve((s1,), (1.0,))[0])
     assert torch.equal(both[1], solve((s1,), (0.5,))[0])
+
+
+def test_first_2n_list_while_another_stream_is_captured():
+    """A program's first 2N list beside a capture on another stream: the capture ends whole, its replays give the
+    eager result, and the list's result is that of a list without a capture."""
+    import torch
+
+    from inductioneq_amd.program import Program
+    from inductioneq_amd.schedules import rk_schedule
+    from test_gpu_node import _stage_case
+    from test_gpu_tiled import _aos
+
+    cfg, B, U = _stage_case("4thOrder", (40, 30, 20), False, True, None, "double")
+    cfg.dt = 1e-5
+    names, nf = rk_schedule("CarpenterKennedy2N54", True, True)
+    side, work = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def solve(capture):
+        prog = Program(cfg)
+        a = [prog.upload_real4(_aos(cfg, B))] + [prog.vector() for _ in range(nf)]
+        a += [prog.upload_real4(_aos(cfg, U)), prog.scalar(1.0), prog.time_buffer()]
+        x, y, g = torch.ones(1000, device="cuda"), torch.zeros(1000, device="cuda"), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(work):
+            prog.use_current_stream()
+        if capture:
+            with torch.cuda.graph(g, stream=side):
+                torch.add(x, 2.0, out=y)
+                prog.run(names, a)
+        else:
+            prog.run(names, a)
+        torch.cuda.synchronize()
+        for k in range(3 if capture else 0):
+            x.fill_(float(k))
+            g.replay()
+            torch.cuda.synchronize()
+            assert bool((y == k + 2.0).all())
+        return a[0].clone()
+
+    assert torch.equal(solve(True), solve(False))

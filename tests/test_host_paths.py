@@ -164,3 +164,17 @@ def test_program_buffers_are_handed_from_stream_to_stream(hip, call):
         assert go(A) == [("record", hex(D)), ("wait", hex(A))]
         assert go(A) == []
     """ % call)
+
+
+def test_the_lists_second_b1_is_allocated_in_relaxed_capture_mode(hip):
+    """A 2N list launches kernels and allocates its second b1 once; the allocation must not end a capture that another
+    stream or thread has begun, which the mode of the calling thread decides.  The mode is as before afterwards."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=10, nz=9)
+        names, nf = rk_schedule("CarpenterKennedy2N54", False, False)
+        assert run(h, names, far(6), (12, 10, 9)) == 0
+        assert [l[-1] for l in log("malloc")] == ["relaxed"]
+        mode = ctypes.c_int(2)
+        H.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
+        assert mode.value == 0
+    """)
