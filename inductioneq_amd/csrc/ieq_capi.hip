@@ -523,8 +523,28 @@ void* b1_copy_for(ieq_program* pr) {
   return pr->b1_copy && pr->shared.enter(pr->stream) ? pr->b1_copy : nullptr;
 }
 
+// Whether the arguments of a time-integrator list that its kernels use (curlB_rho and rho with the Hall term only)
+// are buffers of their own.
+bool args_apart(const ieq_program* pr, void* const* args, int nargs) {
+  const int nf = nargs - 4;
+  if (nf != 2 && nf != 3) return false;
+  const uintptr_t scalar = (uintptr_t)pr->info.stride * pr->info.real_bytes;
+  uintptr_t at[7], end[7];
+  int m = 0;
+  for (int k = 0; k < nargs; ++k) {
+    if ((k == nf || k == nf + 2) && !pr->info.hall) continue;
+    at[m] = (uintptr_t)args[k];
+    end[m] = at[m] + (k == nf + 3 ? 2 * pr->info.real_bytes : k == nf + 2 ? scalar : 3 * scalar);
+    for (int i = 0; i < m; ++i)
+      if (at[i] < end[m] && at[m] < end[i]) return false;
+    ++m;
+  }
+  return true;
+}
+
 // Runs a kernel list.  Neighbouring kernels of the time integrators share a launch where every kernel of the
-// group would be accepted by itself and no value differs: calc_curlB_rho + calc_u; a kernel that only sets the
+// group would be accepted by itself and no value differs (with arguments that share memory the order of the kernels
+// could: those run one by one): calc_curlB_rho + calc_u; a kernel that only sets the
 // stage time and the kernel that reads it; and, on the whole grid, the two halves of a 2N stage (b1' goes to a
 // second copy of b1, in pairs, so that b1 ends where it began).
 template <typename R>
@@ -537,10 +557,11 @@ int run_list_t(ieq_program* pr, const char* const* names, int n, const uint32_t 
   bool all_set = true;
   for (void* a : A) all_set = all_set && a != nullptr;
   const bool modules = pr->has("kernel_time_integrator"), rhs = pr->has("induction_Eq_volume") && pr->has("induction_Eq_surface");
-  const bool in_range = range_ok(pr, g, 0), whole = full_grid(pr, g);
+  const bool in_range = range_ok(pr, g, 0), whole = full_grid(pr, g), apart = all_set && args_apart(pr, args, nargs);
   auto accepted = [&](const char* name) -> const StageDesc* {  // a time-integrator kernel that run_one would launch
+    if (!apart) return nullptr;
     const StageDesc* st = name ? find_stage(name) : nullptr;
-    return st && all_set && modules && (rhs || st->kind != K_STAGE) && nargs == st->nf + 4 && in_range ? st : nullptr;
+    return st && modules && (rhs || st->kind != K_STAGE) && nargs == st->nf + 4 && in_range ? st : nullptr;
   };
   const bool tiled = whole && ieq::tiled_stage_ok(p, ops, (int)sizeof(R));
   const bool node = !(tiled && ieq::tiled_stage_pays(p, ops, (int)sizeof(R)));

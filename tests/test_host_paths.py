@@ -178,3 +178,42 @@ def test_the_lists_second_b1_is_allocated_in_relaxed_capture_mode(hip):
         H.hipThreadExchangeStreamCaptureMode(ctypes.byref(mode))
         assert mode.value == 0
     """)
+
+
+@pytest.mark.parametrize("integrator,field,other", [("SSPRK33", 4, 3), ("SSPRK33", 4, 0), ("SSPRK33", 4, 5),
+                                                    ("CarpenterKennedy2N54", 0, 3), ("CarpenterKennedy2N54", 1, 2)])
+@pytest.mark.parametrize("inside", [0, 4096])
+def test_lists_on_arguments_that_share_memory_run_one_by_one(hip, integrator, field, other, inside):
+    """With two arguments in one buffer, or one that begins inside another, the kernels' order is part of the result:
+    a list launches exactly what its kernels launch one by one."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=10, nz=9, hall=True, testcase="hall_periodic")
+        names, nf = rk_schedule(%r, True, True)
+
+        def kernels(args, names):
+            H.host_hip_clear()
+            for k in names:
+                assert run(h, k, args, (12, 10, 9)) == 0
+            return [l[1] for l in log("launch")]
+
+        args = far(nf + 4)
+        whole = names * 2
+        assert len(kernels(args, [whole])) < len(kernels(args, whole))
+        args[%d] = args[%d] + %d
+        assert kernels(args, [whole]) == kernels(args, whole)
+    """ % (integrator, field, other, inside))
+
+
+def test_unused_arguments_may_share_memory(hip):
+    """Without the Hall term nothing uses curlB_rho and rho: what is passed for them does not keep launches apart."""
+    hostrun(hip, """
+        h = build(opset="4thOrder", nx=12, ny=10, nz=9)
+        names, nf = rk_schedule("CarpenterKennedy2N54", False, False)
+        args = far(6)
+        n = []
+        for a in (args, args[:2] + [args[3], args[3], args[3], args[5]]):
+            H.host_hip_clear()
+            assert run(h, names * 2, a, (12, 10, 9)) == 0
+            n.append(len(log("launch")))
+        assert n[0] == n[1]
+    """)
