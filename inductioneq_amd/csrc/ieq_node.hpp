@@ -35,11 +35,15 @@ __device__ __forceinline__ int node_step(const NodeAxis& a, int k, int periodic)
   return (unsigned)(a.i + k) < (unsigned)a.n ? k : out;
 }
 
-// Value at a byte offset from a component's base; I is unsigned where three components of a field
-// stay below 4 GiB (one 32-bit register per address), long long otherwise.
+// Value at a byte offset from a component's plane; I is unsigned where the plane stays below 4 GiB (one 32-bit
+// register per address), long long otherwise.
 template <typename R, typename I> __device__ __forceinline__ R node_ld(const R* __restrict__ f, I off) {
   return *(const R*)((const char*)f + off);
 }
+template <typename R, typename I> __device__ __forceinline__ void node_st(R* __restrict__ f, I off, R v) {
+  *(R*)((char*)f + off) = v;
+}
+template <typename R> inline bool wide_plane(const Params& p) { return (long long)p.nx * p.ny * (long long)sizeof(R) >= (1LL << 32); }
 
 // First derivative along one axis, not divided by the spacing; `at(k)` is the value k nodes away and
 // T the type it is accumulated in.

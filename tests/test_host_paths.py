@@ -217,3 +217,19 @@ def test_unused_arguments_may_share_memory(hip):
             n.append(len(log("launch")))
         assert n[0] == n[1]
     """)
+
+
+@pytest.mark.parametrize("real,below,above", [("float", (32767, 32768, 9), (32768, 32768, 9)), ("double", (8191, 65536, 9), (8192, 65536, 9))])
+def test_planes_of_4_gib_take_64_bit_offsets(hip, real, below, above):
+    """In-plane byte offsets of 32 bits wrap where a component's plane takes 4 GiB: kernels with 64-bit offsets there."""
+    hostrun(hip, """
+        names = {}
+        for n in (%r, %r, (64, 64, 9)):
+            h = build(real=%r, opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], hall=True, testcase="hall_periodic")
+            H.host_hip_clear()
+            for k in ("calc_curlB_rho_2_3args", "SSPRK33_2b"):
+                assert run(h, k, far(7), n) == 0, lib.ieq_last_error(h)
+            names[n] = {l[1] for l in log("launch")}
+        below, above, small = names.values()
+        assert below == small and not above & small, names
+    """ % (below, above, real))
