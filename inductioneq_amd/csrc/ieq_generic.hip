@@ -20,32 +20,33 @@ constexpr int BX = 64, BY = 4;
 // general row there for all lanes.  One node per thread spends 300 instructions,
 // most of them on rows and indices: 192^3 FP32, 4th order, div B 66 -> 44 us, its norm 112 -> 33, projection 68 -> 41;
 // the four fields of div B once take 23 us as a copy.
-template <typename R, int OPS, bool ADJ> struct Column {
+// I: in-plane byte offsets (ieq_node.hpp).
+template <typename R, int OPS, bool ADJ, typename I> struct Column {
   using O = Op<OPS>;
   static constexpr int W = O::W, C = (W - 1) / 2;
-  unsigned o;  // in-plane byte offset of the nodes
+  I o;  // in-plane byte offset of the nodes
   bool mx, my;
   R cx[W], cy[W];
-  unsigned ox[W], oy[W];
+  I ox[W], oy[W];
   __device__ static double coef(int row, int k) { return ADJ ? O::dadj(row, k) : O::d(row, k); }
   __device__ __forceinline__ void init(const Params& p, int ix, int iy) {
     const NodeAxis ax = node_axis<OPS>(ix, p.nx, p.periodic), ay = node_axis<OPS>(iy, p.ny, p.periodic);
-    const unsigned RB = sizeof(R);
-    o = (unsigned)(ix + p.nx * iy) * RB;
+    const I RB = sizeof(R);
+    o = ((I)ix + (I)p.nx * (I)iy) * RB;
     mx = __all(ax.mid);
     my = __all(ay.mid);
 #pragma unroll
     for (int k = 0; k < W; ++k) {
       cx[k] = (R)coef(mx ? O::NB : ax.row, k);
       cy[k] = (R)coef(my ? O::NB : ay.row, k);
-      ox[k] = o + (unsigned)node_step(ax, k - C, p.periodic) * RB;
-      oy[k] = o + (unsigned)(node_step(ay, k - C, p.periodic) * p.nx) * RB;
+      ox[k] = o + (I)node_step(ax, k - C, p.periodic) * RB;
+      oy[k] = o + (I)node_step(ay, k - C, p.periodic) * (I)p.nx * RB;
     }
   }
   // MX, MY, MZ: the central row is taken along x, y, z (compile-time, so that the loads of all directions of a
   // node are one run without branches; with a branch per direction a plane waits for three load latencies).
   // f: the component's plane iz.
-  template <bool MID> __device__ __forceinline__ R line(const Params& p, const R* f, const R (&c)[W], const unsigned (&off)[W], int d) const {
+  template <bool MID> __device__ __forceinline__ R line(const Params& p, const R* f, const R (&c)[W], const I (&off)[W], int d) const {
     R acc = R(0);
 #pragma unroll
     for (int k = 0; k < W; ++k) {
@@ -101,13 +102,35 @@ template <typename R, int OPS, bool ADJ> struct Column {
 };
 
 // A block of the column kernels: 256 consecutive nodes of an xy-plane of the NDRange (full lanes whatever the
-// sizes) and `zc` planes, blocks in contiguous ranges per XCD.
+// sizes) and `zc` planes; blocks in contiguous ranges per XCD, in rows of at most kRow (HIP takes fewer than 2^32
+// threads in a dimension).
+constexpr unsigned kRow = 1 << 22;
+struct ColumnGrid {
+  long long gxy;           // nodes of the NDRange in a plane
+  int gx, gz, segs, zc, blocks;  // ... in x and z; runs of 256 in a plane, planes of a block, blocks
+  dim3 rows() const { return blocks <= (int)kRow ? dim3((unsigned)blocks) : dim3(kRow, ((unsigned)blocks + kRow - 1) / kRow); }
+};
+// Planes per block: about 4096 blocks, so that the chip is full and a thread still has a few planes to share its
+// rows between.
+ColumnGrid column_grid(const uint32_t g[3]) {
+  ColumnGrid c;
+  c.gxy = (long long)g[0] * g[1];
+  c.gx = (int)g[0];
+  c.gz = (int)g[2];
+  c.segs = (int)((c.gxy + 255) / 256);
+  c.zc = (int)std::max(1LL, std::min(16LL, (long long)c.segs * c.gz / 4096));
+  c.blocks = c.segs * ((c.gz + c.zc - 1) / c.zc);
+  return c;
+}
 #define IEQ_COLUMN_PREAMBLE(OFF)                                                                              \
-  const int segs = (int)((g.x * g.y + 255) / 256), tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;   \
-  const uint32_t jt = (uint32_t)(tile - ch * segs) * 256 + threadIdx.x;                                       \
-  if (jt >= g.x * g.y) return;                                                                                \
-  const int ix = (int)(jt % g.x) + (OFF), iy = (int)(jt / g.x) + (OFF);                                       \
-  const int z0 = ch * zc + (OFF), z1 = min(z0 + zc, (int)g.z + (OFF));                                        \
+  const int linear = (int)(blockIdx.y * kRow + blockIdx.x);                                                   \
+  if (linear >= cg.blocks) return;                                                                            \
+  const int tile = xcd_tile(linear, cg.blocks), ch = tile / cg.segs;                                          \
+  using P = std::conditional_t<std::is_same_v<I, unsigned>, uint32_t, uint64_t>;                              \
+  const P jt = (P)(tile - ch * cg.segs) * 256 + threadIdx.x, gx = (P)cg.gx;                                   \
+  if (jt >= (P)cg.gxy) return;                                                                                \
+  const int ix = (int)(jt % gx) + (OFF), iy = (int)(jt / gx) + (OFF);                                         \
+  const int z0 = ch * cg.zc + (OFF), z1 = min(z0 + cg.zc, cg.gz + (OFF));                                     \
   const long long S = p.stride, nxy = (long long)p.nx * p.ny;                                                 \
   (void)S; (void)nxy;
 
@@ -178,38 +201,38 @@ template <typename R> __global__ __launch_bounds__(BX* BY) void k_init(Params p,
   else st3(f, S, idx, b_analytical<R>(p, ix, iy, iz, time[0]));
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(256) void k_div(Params p, Range g, int zc, const R* b, R* out, int off) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div(Params p, ColumnGrid cg, const R* b, R* out, int off) {
   IEQ_COLUMN_PREAMBLE(off)
-  Column<R, OPS, false> c;
+  Column<R, OPS, false, I> c;
   c.init(p, ix, iy);
   c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
-    sto(out + iz * nxy, c.o, c.template div<x.value, y.value, z.value>(p, b + iz * nxy, iz));
+    node_st(out + iz * nxy, c.o, c.template div<x.value, y.value, z.value>(p, b + iz * nxy, iz));
   });
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(256) void k_curl(Params p, Range g, int zc, const R* b, R* out) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_curl(Params p, ColumnGrid cg, const R* b, R* out) {
   IEQ_COLUMN_PREAMBLE(0)
-  Column<R, OPS, false> c;
+  Column<R, OPS, false, I> c;
   c.init(p, ix, iy);
   c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {  // SBP_operator.cl:126-135
     const R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
     R* f = out + iz * nxy;
-    sto(f, c.o, c.template dy<y.value>(p, bz) - c.template dz<z.value>(p, by, iz));
-    sto(f + S, c.o, c.template dz<z.value>(p, bx, iz) - c.template dx<x.value>(p, bz));
-    sto(f + 2 * S, c.o, c.template dx<x.value>(p, by) - c.template dy<y.value>(p, bx));
+    node_st(f, c.o, c.template dy<y.value>(p, bz) - c.template dz<z.value>(p, by, iz));
+    node_st(f + S, c.o, c.template dz<z.value>(p, bx, iz) - c.template dx<x.value>(p, bz));
+    node_st(f + 2 * S, c.o, c.template dx<x.value>(p, by) - c.template dy<y.value>(p, bx));
   });
 }
 
-template <typename R, int OPS> __global__ __launch_bounds__(256) void k_grad(Params p, Range g, int zc, const R* f, R* out) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_grad(Params p, ColumnGrid cg, const R* f, R* out) {
   IEQ_COLUMN_PREAMBLE(0)
-  Column<R, OPS, false> c;
+  Column<R, OPS, false, I> c;
   c.init(p, ix, iy);
   c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
     const R* fz = f + iz * nxy;
     R* o = out + iz * nxy;
-    sto(o, c.o, c.template dx<x.value>(p, fz));
-    sto(o + S, c.o, c.template dy<y.value>(p, fz));
-    sto(o + 2 * S, c.o, c.template dz<z.value>(p, fz, iz));
+    node_st(o, c.o, c.template dx<x.value>(p, fz));
+    node_st(o + S, c.o, c.template dy<y.value>(p, fz));
+    node_st(o + 2 * S, c.o, c.template dz<z.value>(p, fz, iz));
   });
 }
 
@@ -217,14 +240,16 @@ template <typename R, int OPS> __global__ __launch_bounds__(256) void k_grad(Par
 // divergence in REAL as calc_div stores it, weights, squares and sums in double.  One partial per block, at
 // most kNormBlocks of them: runs of a plane beyond that many are walked with a stride.
 constexpr int kNormBlocks = 1024;
-template <typename R, int OPS> __global__ __launch_bounds__(256) void k_div_norm(Params p, int segs, int zc, const R* b, double* part) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div_norm(Params p, int segs, int zc, const R* b, double* part) {
   using O = Op<OPS>;
-  const int nxy = p.nx * p.ny, tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;
+  using P = std::conditional_t<std::is_same_v<I, unsigned>, int, long long>;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;
+  const P nxy = (P)p.nx * p.ny;
   const int z0 = ch * zc, z1 = min(z0 + zc, p.nz);
   double acc = 0.0;
-  for (int j = (tile - ch * segs) * 256 + (int)threadIdx.x; j < nxy; j += segs * 256) {
-    const int ix = j % p.nx, iy = j / p.nx;
-    Column<R, OPS, false> c;
+  for (P j = (tile - ch * segs) * 256 + (int)threadIdx.x; j < nxy; j += segs * 256) {
+    const int ix = (int)(j % p.nx), iy = (int)(j / p.nx);
+    Column<R, OPS, false, I> c;
     c.init(p, ix, iy);
     const double fxy = (p.dx / O::minv(bound_row(ix, p.nx, O::NB, p.periodic))) * (p.dy / O::minv(bound_row(iy, p.ny, O::NB, p.periodic)));
     c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
@@ -277,19 +302,19 @@ template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_lap(P
 }
 
 // projector_divcleaning (kernel_div_cleaning.cl:96-109): B +/- grad(phi), .xyz only
-template <typename R, int OPS> __global__ __launch_bounds__(256) void k_proj(Params p, Range g, int zc, R* b, const R* phi) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_proj(Params p, ColumnGrid cg, R* b, const R* phi) {
   IEQ_COLUMN_PREAMBLE(0)
   auto apply = [&](auto adj, R sgn) {
-    Column<R, OPS, decltype(adj)::value> c;
+    Column<R, OPS, decltype(adj)::value, I> c;
     c.init(p, ix, iy);
     c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
       const R* f = phi + iz * nxy;
       R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
       const R vx = node_ld(bx, c.o), vy = node_ld(by, c.o), vz = node_ld(bz, c.o);
       const R dx = c.template dx<x.value>(p, f), dy = c.template dy<y.value>(p, f), dz = c.template dz<z.value>(p, f, iz);
-      sto(bx, c.o, vx + sgn * dx);
-      sto(by, c.o, vy + sgn * dy);
-      sto(bz, c.o, vz + sgn * dz);
+      node_st(bx, c.o, vx + sgn * dx);
+      node_st(by, c.o, vy + sgn * dy);
+      node_st(bz, c.o, vz + sgn * dz);
     });
   };
   if (p.laplace == 2) apply(std::true_type{}, R(-1));
@@ -371,16 +396,6 @@ template <typename R> __global__ void k_soa_to_aos(const R* soa, R* aos, long lo
   aos[4 * i + 3] = R(0);
 }
 
-// Planes per block and blocks of the column kernels: about 4096 blocks, so that the chip is full and a thread
-// still has a few planes to share its rows between.
-int column_zc(Range g) {
-  const long long runs = (long long)((g.x * g.y + 255) / 256) * g.z;
-  return (int)std::max(1LL, std::min(16LL, runs / 4096));
-}
-unsigned column_blocks(Range g) {
-  const int zc = column_zc(g);
-  return ((g.x * g.y + 255) / 256) * ((g.z + zc - 1) / zc);
-}
 dim3 grid_of(Range g) { return dim3((g.x + BX - 1) / BX, (g.y + BY - 1) / BY, g.z); }
 
 }  // namespace
@@ -397,6 +412,9 @@ dim3 grid_of(Range g) { return dim3((g.x + BX - 1) / BX, (g.y + BY - 1) / BY, g.
     case 4: { constexpr int OPS = 4; CALL; } break; \
     default: { constexpr int OPS = 5; CALL; } break; \
   }
+
+#define IEQ_PLANE_SWITCH(R, p, CALL) \
+  if (wide_plane<R>(p)) { using I = long long; CALL } else { using I = unsigned; CALL }
 
 template <typename R>
 void gen_update_2r(const Params& p, hipStream_t s, const uint32_t g[3], R* X, R* O, const R* D, R a, R b, R* time, double tc) {
@@ -425,26 +443,26 @@ template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32
 }
 
 template <typename R> void gen_div(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out, int off) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_div<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out, off)))
+  const ColumnGrid cg = column_grid(g);
+  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_div<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out, off))))
 }
 
 template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s, const R* b, double* part, double* out) {
   const long long runs = ((long long)p.nx * p.ny + 255) / 256;
   const int segs = (int)std::min<long long>(runs, kNormBlocks), most = kNormBlocks / segs, zc = (p.nz + most - 1) / most;
   const int nb = segs * ((p.nz + zc - 1) / zc);
-  IEQ_OPS_SWITCH(ops, (k_div_norm<R, OPS><<<nb, 256, 0, s>>>(p, segs, zc, b, part)))
+  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_div_norm<R, OPS, I><<<nb, 256, 0, s>>>(p, segs, zc, b, part))))
   k_sum<<<1, 256, 0, s>>>(part, nb, out);
 }
 
 template <typename R> void gen_curl(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_curl<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, out)))
+  const ColumnGrid cg = column_grid(g);
+  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_curl<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out))))
 }
 
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_grad<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), f, out)))
+  const ColumnGrid cg = column_grid(g);
+  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_grad<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, f, out))))
 }
 
 template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
@@ -453,8 +471,8 @@ template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, cons
 }
 
 template <typename R> void gen_proj(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* b, const R* phi) {
-  Range r{g[0], g[1], g[2]};
-  IEQ_OPS_SWITCH(ops, (k_proj<R, OPS><<<column_blocks(r), 256, 0, s>>>(p, r, column_zc(r), b, phi)))
+  const ColumnGrid cg = column_grid(g);
+  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_proj<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi))))
 }
 
 template <typename R> void gen_axpy(const Params& p, hipStream_t s, const uint32_t g[3], R* x, const R* y, const R* a, int xpay) {

@@ -79,3 +79,24 @@ def test_stage_kernels_on_wide_planes():
             _same(J, out["J"], n, 3)
             del J
             _same(res, out["res"], n, 3)
+
+
+def test_column_kernels_on_wide_planes():
+    import torch
+
+    from inductioneq_amd.program import Program
+
+    for name, parts, res in (("calc_div", 3, 1), ("calc_curl", 3, 3), ("calc_grad", 1, 3)):
+        small = None
+        for n in (TILE, WIDE):
+            prog = Program(_cfg(n))
+            f = _field(prog, n, _tile(parts, 4))
+            out = prog.vector() if res == 3 else prog.scalar()
+            prog.run(name, [f, out])
+            torch.cuda.synchronize()
+            del f
+            if n == TILE:
+                small = out
+            else:
+                _same(out, small, n, res)
+            del out

@@ -225,11 +225,32 @@ def test_planes_of_4_gib_take_64_bit_offsets(hip, real, below, above):
     hostrun(hip, """
         names = {}
         for n in (%r, %r, (64, 64, 9)):
-            h = build(real=%r, opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], hall=True, testcase="hall_periodic")
+            h = build(real=%r, opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], hall=True, testcase="hall_periodic",
+                      laplace="WIDE_STENCIL_LNS")
             H.host_hip_clear()
             for k in ("calc_curlB_rho_2_3args", "SSPRK33_2b"):
                 assert run(h, k, far(7), n) == 0, lib.ieq_last_error(h)
+            for k in ("calc_div", "calc_curl", "calc_grad", "projector_divcleaning"):
+                assert run(h, k, far(2), n) == 0, lib.ieq_last_error(h)
             names[n] = {l[1] for l in log("launch")}
         below, above, small = names.values()
         assert below == small and not above & small, names
     """ % (below, above, real))
+
+
+@pytest.mark.parametrize("n", [(65600, 65600, 2), (1024, 1024, 1024), (100, 90, 80)])
+def test_column_kernels_launch_shape(hip, n):
+    """Runs of 256 nodes of a plane times z-chunks, in rows that HIP takes (4.3e9 nodes a plane: 1.7e7 runs)."""
+    hostrun(hip, """
+        n = %r
+        h = build(real="float", opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], testcase="rotation_2D", laplace="WIDE_STENCIL_LNS")
+        for k in ("calc_div", "calc_curl", "calc_grad", "projector_divcleaning"):
+            H.host_hip_clear()
+            assert run(h, k, far(2), n) == 0, lib.ieq_last_error(h)
+            (l,) = log("launch", "refused")
+            x, y, z, threads = [int(v) for v in l[2:6]]
+            runs = (n[0] * n[1] + 255) // 256
+            zc = max(1, min(16, runs * n[2] // 4096))
+            need = runs * -(-n[2] // zc)
+            assert z == 1 and threads == 256 and need <= x * y < need + x, (x, y, need)
+    """ % (n,))
