@@ -237,19 +237,18 @@ template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) voi
 }
 
 // Partial sums of the squared SBP norm of div B (calc_div + norm2_S, kernel_operator.cl:98-155): the
-// divergence in REAL as calc_div stores it, weights, squares and sums in double.  One partial per block, at
+// divergence in REAL as calc_div stores it, weights, squares and sums in double, of a component below 2 GiB (its
+// caller's limit).  One partial per block, at
 // most kNormBlocks of them: runs of a plane beyond that many are walked with a stride.
 constexpr int kNormBlocks = 1024;
-template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div_norm(Params p, int segs, int zc, const R* b, double* part) {
+template <typename R, int OPS> __global__ __launch_bounds__(256) void k_div_norm(Params p, int segs, int zc, const R* b, double* part) {
   using O = Op<OPS>;
-  using P = std::conditional_t<std::is_same_v<I, unsigned>, int, long long>;
-  const int tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;
-  const P nxy = (P)p.nx * p.ny;
+  const int nxy = p.nx * p.ny, tile = xcd_tile(blockIdx.x, gridDim.x), ch = tile / segs;
   const int z0 = ch * zc, z1 = min(z0 + zc, p.nz);
   double acc = 0.0;
-  for (P j = (tile - ch * segs) * 256 + (int)threadIdx.x; j < nxy; j += segs * 256) {
-    const int ix = (int)(j % p.nx), iy = (int)(j / p.nx);
-    Column<R, OPS, false, I> c;
+  for (int j = (tile - ch * segs) * 256 + (int)threadIdx.x; j < nxy; j += segs * 256) {
+    const int ix = j % p.nx, iy = j / p.nx;
+    Column<R, OPS, false, unsigned> c;
     c.init(p, ix, iy);
     const double fxy = (p.dx / O::minv(bound_row(ix, p.nx, O::NB, p.periodic))) * (p.dy / O::minv(bound_row(iy, p.ny, O::NB, p.periodic)));
     c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
@@ -451,7 +450,7 @@ template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s
   const long long runs = ((long long)p.nx * p.ny + 255) / 256;
   const int segs = (int)std::min<long long>(runs, kNormBlocks), most = kNormBlocks / segs, zc = (p.nz + most - 1) / most;
   const int nb = segs * ((p.nz + zc - 1) / zc);
-  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_div_norm<R, OPS, I><<<nb, 256, 0, s>>>(p, segs, zc, b, part))))
+  IEQ_OPS_SWITCH(ops, (k_div_norm<R, OPS><<<nb, 256, 0, s>>>(p, segs, zc, b, part)))
   k_sum<<<1, 256, 0, s>>>(part, nb, out);
 }
 
