@@ -50,22 +50,26 @@ __device__ inline double wave_sum(double v) {
 // every plane of the chunk, so their rows are found once per thread, and the z row is uniform in a wave.
 // 128^3 FP32, 4th order, with an analytic field: 31 us, against 72 us with a 64-bit division and rolled
 // table rows per node.  TC is the testcase whose analytic field the error is taken against (-1: none):
-// with all of them in one kernel the code of the other seven holds 235 registers (44 us).
-template <typename R, int OPS, int TC>
+// with all of them in one kernel the code of the other seven holds 235 registers (44 us).  Numbers of a plane's
+// nodes are P: 64 bits, and then the program's testcase (kAnyCase), only where 32 do not hold them.
+constexpr int kAnyCase = -2;
+template <typename R, int OPS, int TC, typename P>
 __global__ __launch_bounds__(kDiagThreads) void k_diag(Params p, DiagSplit sp, const R* b, double t, double* part) {
   using O = Op<OPS>;
-  const int nxy = p.nx * p.ny, per = p.periodic;
+  const P nxy = (P)p.nx * p.ny;
+  const int per = p.periodic;
   const long long S = p.stride;
   const double ih[3] = {1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
   const int seg0 = (int)blockIdx.x % sp.segs, z0 = ((int)blockIdx.x / sp.segs) * sp.zc, z1 = min(z0 + sp.zc, p.nz);
-  p.testcase = TC;
-  const double st = TC >= 0 ? sin(t) : 0.0, ct = TC >= 0 ? cos(t) : 0.0;
+  if (TC != kAnyCase) p.testcase = TC;
+  const bool analytic = TC >= 0 || (TC == kAnyCase && p.testcase >= 0);
+  const double st = analytic ? sin(t) : 0.0, ct = analytic ? cos(t) : 0.0;
   __shared__ NodeTable<double, OPS> tab;
   tab.load(threadIdx.x, kDiagThreads);
   __syncthreads();
   double acc[3] = {0.0, 0.0, 0.0};
-  for (int j = seg0 * kDiagThreads + (int)threadIdx.x; j < nxy; j += sp.segs * kDiagThreads) {
-    const int iy = j / p.nx, ix = j - iy * p.nx;
+  for (P j = seg0 * kDiagThreads + (int)threadIdx.x; j < nxy; j += sp.segs * kDiagThreads) {
+    const int iy = (int)(j / p.nx), ix = (int)(j - (P)iy * p.nx);
     const NodeAxis ax = node_axis<OPS>(ix, p.nx, per), ay = node_axis<OPS>(iy, p.ny, per);
     const bool mxy = __all(ax.mid && ay.mid);
     const double fxy = (p.dx / O::minv(ax.row)) * (p.dy / O::minv(ay.row));
@@ -81,16 +85,16 @@ __global__ __launch_bounds__(kDiagThreads) void k_diag(Params p, DiagSplit sp, c
       double dx, dy, dz;
       if (mxy && az.mid) {
         dx = node_deriv_mid<double, OPS>([&](int k) { return (double)fx[j + node_step(ax, k, per)]; });
-        dy = node_deriv_mid<double, OPS>([&](int k) { return (double)fy[j + p.nx * node_step(ay, k, per)]; });
+        dy = node_deriv_mid<double, OPS>([&](int k) { return (double)fy[j + (P)p.nx * node_step(ay, k, per)]; });
         dz = node_deriv_mid<double, OPS>([&](int k) { return (double)fz[j + (long long)nxy * node_step(az, k, per)]; });
       } else {
         dx = node_deriv_row<double, OPS>(tab, ax, per, [&](int st) { return (double)fx[j + st]; });
-        dy = node_deriv_row<double, OPS>(tab, ay, per, [&](int st) { return (double)fy[j + p.nx * st]; });
+        dy = node_deriv_row<double, OPS>(tab, ay, per, [&](int st) { return (double)fy[j + (P)p.nx * st]; });
         dz = node_deriv_row<double, OPS>(tab, az, per, [&](int st) { return (double)fz[j + (long long)nxy * st]; });
       }
       const double dv = dx * ih[0] + dy * ih[1] + dz * ih[2];
       acc[1] += fac * (dv * dv);
-      if constexpr (TC >= 0) {
+      if (analytic) {
         const V3<double> a = b_analytical<double>(p, ix, iy, iz, t, st, ct);
         const double ex = bx - a.x, ey = by - a.y, ez = bz - a.z;
         acc[2] += fac * (ex * ex + ey * ey + ez * ez);
@@ -133,27 +137,28 @@ __global__ __launch_bounds__(kDiagThreads) void k_diag_sum(const double* part, i
                                                                             : sqrt(fmax(s, 0.0));
 }
 
-template <typename R, int OPS> const void* diag_kernel_t(int tc) {
+template <typename R, int OPS> const void* diag_kernel_t(int tc, bool wide) {
+  if (wide) return reinterpret_cast<const void*>(&k_diag<R, OPS, kAnyCase, long long>);
   switch (tc) {
-    case TC_ROTATION_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_2D>);
-    case TC_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_3D>);
-    case TC_HALL_PERIODIC: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_PERIODIC>);
-    case TC_HALL_TRAVELLING_WAVE: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_TRAVELLING_WAVE>);
-    case TC_CONFINED_DOMAIN: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_CONFINED_DOMAIN>);
-    case TC_ALFVEN_PERIODIC_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ALFVEN_PERIODIC_2D>);
-    case TC_GAUSSIAN_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_GAUSSIAN_ROTATION_3D>);
-    case TC_UNIFORM_FLOW: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_UNIFORM_FLOW>);
-    default: return reinterpret_cast<const void*>(&k_diag<R, OPS, -1>);
+    case TC_ROTATION_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_2D, int>);
+    case TC_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ROTATION_3D, int>);
+    case TC_HALL_PERIODIC: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_PERIODIC, int>);
+    case TC_HALL_TRAVELLING_WAVE: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_HALL_TRAVELLING_WAVE, int>);
+    case TC_CONFINED_DOMAIN: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_CONFINED_DOMAIN, int>);
+    case TC_ALFVEN_PERIODIC_2D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_ALFVEN_PERIODIC_2D, int>);
+    case TC_GAUSSIAN_ROTATION_3D: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_GAUSSIAN_ROTATION_3D, int>);
+    case TC_UNIFORM_FLOW: return reinterpret_cast<const void*>(&k_diag<R, OPS, TC_UNIFORM_FLOW, int>);
+    default: return reinterpret_cast<const void*>(&k_diag<R, OPS, -1, int>);
   }
 }
-template <typename R> const void* diag_kernel(int ops, int tc) {
+template <typename R> const void* diag_kernel(int ops, int tc, bool wide) {
   switch (ops) {
-    case 0: return diag_kernel_t<R, 0>(tc);
-    case 1: return diag_kernel_t<R, 1>(tc);
-    case 2: return diag_kernel_t<R, 2>(tc);
-    case 3: return diag_kernel_t<R, 3>(tc);
-    case 4: return diag_kernel_t<R, 4>(tc);
-    default: return diag_kernel_t<R, 5>(tc);
+    case 0: return diag_kernel_t<R, 0>(tc, wide);
+    case 1: return diag_kernel_t<R, 1>(tc, wide);
+    case 2: return diag_kernel_t<R, 2>(tc, wide);
+    case 3: return diag_kernel_t<R, 3>(tc, wide);
+    case 4: return diag_kernel_t<R, 4>(tc, wide);
+    default: return diag_kernel_t<R, 5>(tc, wide);
   }
 }
 
@@ -169,8 +174,9 @@ hipError_t diag_launch(const Params& p, int ops, hipStream_t s, const R* b, doub
                        double* out_dev) {
   const DiagSplit sp = diag_split(p);
   const int nblk = sp.segs * sp.chunks;
-  const void* k = diag_kernel<R>(ops, analytic ? p.testcase : -1);
   Params q = p;
+  if (!analytic) q.testcase = -1;
+  const void* k = diag_kernel<R>(ops, q.testcase, (long long)p.nx * p.ny >= (1LL << 30));
   DiagSplit split = sp;
   void* kargs[5] = {(void*)&q, (void*)&split, (void*)&b, (void*)&t, (void*)&part};
   const hipError_t e = hipLaunchKernel(k, dim3(nblk), dim3(kDiagThreads), kargs, 0, s);

@@ -100,3 +100,38 @@ def test_column_kernels_on_wide_planes():
             else:
                 _same(out, small, n, res)
             del out
+
+
+@pytest.mark.parametrize("analytic", [0, 1])
+def test_diagnostics_on_planes_of_2_to_the_31_nodes(analytic):
+    """Sums over the tiles are the tile's times their number (1e-9: up to 4e9 equal terms in another order), the norms
+    its square root; the error is against a field of the coordinates, so there the whole is compared with four parts of
+    it that do not take the wide kernel: quarters of the y range, each with its coordinates."""
+    import math
+
+    import torch
+
+    from inductioneq_amd.program import Program
+
+    n = (46352, 46336, 2)  # 2.148e9 nodes a plane
+    tile = _tile(3, 5)
+
+    def diag(n, **kw):
+        cfg = _cfg(n)
+        for k, v in kw.items():
+            setattr(cfg, k, v)
+        prog = Program(cfg)
+        d = prog.diagnostics(_field(prog, n, tile), 0.0)
+        torch.cuda.empty_cache()
+        return d
+
+    whole = diag(n)
+    if not analytic:
+        one, m = diag(TILE), (n[0] // 16) * (n[1] // 8)
+        assert abs(whole["energy"] - m * one["energy"]) <= 1e-9 * whole["energy"]
+        assert abs(whole["divergence_norm"] - math.sqrt(m) * one["divergence_norm"]) <= 1e-9 * whole["divergence_norm"]
+    else:
+        half = (n[0], n[1] // 4, n[2])
+        parts = [diag(half, ymin=k * half[1] * 0.2)["error_norm"] for k in range(4)]
+        want = math.sqrt(sum(p * p for p in parts))
+        assert want > 0 and abs(whole["error_norm"] - want) <= 1e-9 * want
