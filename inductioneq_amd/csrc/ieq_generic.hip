@@ -210,19 +210,6 @@ template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) voi
   });
 }
 
-template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_curl(Params p, ColumnGrid cg, const R* b, R* out) {
-  IEQ_COLUMN_PREAMBLE(0)
-  Column<R, OPS, false, I> c;
-  c.init(p, ix, iy);
-  c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {  // SBP_operator.cl:126-135
-    const R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
-    R* f = out + iz * nxy;
-    node_st(f, c.o, c.template dy<y.value>(p, bz) - c.template dz<z.value>(p, by, iz));
-    node_st(f + S, c.o, c.template dz<z.value>(p, bx, iz) - c.template dx<x.value>(p, bz));
-    node_st(f + 2 * S, c.o, c.template dx<x.value>(p, by) - c.template dy<y.value>(p, bx));
-  });
-}
-
 template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_grad(Params p, ColumnGrid cg, const R* f, R* out) {
   IEQ_COLUMN_PREAMBLE(0)
   Column<R, OPS, false, I> c;
@@ -454,11 +441,6 @@ template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s
   k_sum<<<1, 256, 0, s>>>(part, nb, out);
 }
 
-template <typename R> void gen_curl(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out) {
-  const ColumnGrid cg = column_grid(g);
-  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_curl<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out))))
-}
-
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
   const ColumnGrid cg = column_grid(g);
   IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_grad<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, f, out))))
@@ -500,7 +482,6 @@ template <typename R> void gen_soa_to_aos(hipStream_t s, const R* soa, R* aos, l
   template void gen_init<R>(const Params&, hipStream_t, const uint32_t*, R*, int, const R*);                                 \
   template void gen_div<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*, int);                             \
   template void gen_div_norm2<R>(const Params&, int, hipStream_t, const R*, double*, double*);                              \
-  template void gen_curl<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                 \
   template void gen_grad<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                 \
   template void gen_lap<R>(const Params&, int, hipStream_t, const uint32_t*, const R*, R*);                                  \
   template void gen_proj<R>(const Params&, int, hipStream_t, const uint32_t*, R*, const R*);                                 \

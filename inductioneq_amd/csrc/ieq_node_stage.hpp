@@ -25,8 +25,8 @@ template <typename R>
 hipError_t node_stage(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* out, const R* P, R cP, const R* Q, R cQ,
                       const R* Y, R cD, const R* J, const R* u, const NodeTime<R>& t, R* b1 = nullptr, R cB = R(0));
 
-// Enqueue J = curl B / rho (J non-null; calc_curlB_rho_*, kernel_time_integrator.cl:136-208) and u =
-// u_analytical at the stage time (u non-null; calc_u_*, :84-134) on the nodes [0, g).
+// Enqueue J = curl B / rho (J non-null; calc_curlB_rho_*, kernel_time_integrator.cl:136-208; rho null: curl B)
+// and u = u_analytical at the stage time (u non-null; calc_u_*, :84-134) on the nodes [0, g).
 template <typename R>
 hipError_t node_pre(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* J, const R* rho, R* u,
                     const NodeTime<R>& t);
