@@ -1,5 +1,5 @@
-// Reference-schedule kernels other than the stages, curl B / rho and calc_u (ieq_node_stage.inc): SBP operators
-// down a column of planes, and one work-item per node for the rest.  These back the reference kernel names
+// Reference-schedule kernels other than the stages, the curls and calc_u (ieq_node_stage.inc): SBP operators down a
+// column of planes or with a thread per node, and one work-item per node for the rest.  These back the reference kernel names
 // accepted by ieq_run(); the fused kernels in ieq_fused.hip replace the hot ones.
 #include <algorithm>
 #include <type_traits>
@@ -17,9 +17,9 @@ constexpr int BX = 64, BY = 4;
 // Derivatives of one component (diff_x/y/z, SBP_operator.cl:12-51) or their M-adjoints at the nodes of a
 // column (fixed x and y, the planes of a chunk): the rows and neighbour offsets along x and y are found
 // once per thread, those along z are uniform in a wave.  A wave with a node near an x (y) face takes its
-// general row there for all lanes.  One node per thread spends 300 instructions,
-// most of them on rows and indices: 192^3 FP32, 4th order, div B 66 -> 44 us, its norm 112 -> 33, projection 68 -> 41;
-// the four fields of div B once take 23 us as a copy.
+// general row there for all lanes.  With rows and indices looked up per node a thread spends 300 instructions:
+// 192^3 FP32, 4th order, div B 63 -> 33 us, its norm 112 -> 33, projection 67 -> 38; the four fields of div B once take
+// 23 us as a copy.
 // I: in-plane byte offsets (ieq_node.hpp).
 template <typename R, int OPS, bool ADJ, typename I> struct Column {
   using O = Op<OPS>;
@@ -110,15 +110,15 @@ struct ColumnGrid {
   int gx, gz, segs, zc, blocks;  // ... in x and z; runs of 256 in a plane, planes of a block, blocks
   dim3 rows() const { return blocks <= (int)kRow ? dim3((unsigned)blocks) : dim3(kRow, ((unsigned)blocks + kRow - 1) / kRow); }
 };
-// Planes per block: about 4096 blocks, so that the chip is full and a thread still has a few planes to share its
-// rows between.
-ColumnGrid column_grid(const uint32_t g[3]) {
+// Planes per block, at most `most`: about 4096 blocks, so that the chip is full and a thread still has a few planes to
+// share its rows between.
+ColumnGrid column_grid(const uint32_t g[3], long long most) {
   ColumnGrid c;
   c.gxy = (long long)g[0] * g[1];
   c.gx = (int)g[0];
   c.gz = (int)g[2];
   c.segs = (int)((c.gxy + 255) / 256);
-  c.zc = (int)std::max(1LL, std::min(16LL, (long long)c.segs * c.gz / 4096));
+  c.zc = (int)std::max(1LL, std::min(most, (long long)c.segs * c.gz / 4096));
   c.blocks = c.segs * ((c.gz + c.zc - 1) / c.zc);
   return c;
 }
@@ -201,7 +201,7 @@ template <typename R> __global__ __launch_bounds__(BX* BY) void k_init(Params p,
   else st3(f, S, idx, b_analytical<R>(p, ix, iy, iz, time[0]));
 }
 
-template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div(Params p, ColumnGrid cg, const R* b, R* out, int off) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div_column(Params p, ColumnGrid cg, const R* b, R* out, int off) {
   IEQ_COLUMN_PREAMBLE(off)
   Column<R, OPS, false, I> c;
   c.init(p, ix, iy);
@@ -210,7 +210,7 @@ template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) voi
   });
 }
 
-template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_grad(Params p, ColumnGrid cg, const R* f, R* out) {
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_grad_column(Params p, ColumnGrid cg, const R* f, R* out) {
   IEQ_COLUMN_PREAMBLE(0)
   Column<R, OPS, false, I> c;
   c.init(p, ix, iy);
@@ -223,6 +223,75 @@ template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) voi
   });
 }
 
+// The derivatives along x, y and z of fx, fy and fz (a node's plane of a component each) with a thread per node: rows of
+// the table from LDS where a wave has a boundary row.
+template <typename R, int OPS, bool ADJ, int D, bool MID, typename I>
+__device__ __forceinline__ R line_deriv(const Params& p, const NodeAxis& A, const R* f, I o, R* tab) {
+  using O = Op<OPS>;
+  constexpr int W = O::W, C = (W - 1) / 2, NB = O::NB;
+  const long long nxy = (long long)p.nx * p.ny;
+  const bool mid = MID || (D == 2 ? A.mid : (bool)__all(A.mid));
+  if (D != 2 && !mid) {
+    for (int i = (int)threadIdx.x & 63; i < (2 * NB + 1) * W; i += 64) tab[i] = (R)(ADJ ? O::dadj(0, i) : O::d(0, i));
+    __builtin_amdgcn_wave_barrier();
+  }
+  R acc = R(0);
+  auto at = [&](int step) {
+    return D == 2 ? node_ld(f + (long long)step * nxy, o) : node_ld(f, o + (D == 0 ? (I)step : (I)step * (I)p.nx) * (I)sizeof(R));
+  };
+  if (mid) {
+#pragma unroll
+    for (int k = -C; k <= C; ++k) {
+      const double m = ADJ ? O::dadj(NB, C + k) : O::d(NB, C + k);
+      if (m != 0.0) acc = acc + (R)m * at(node_step(A, k, p.periodic));
+    }
+  } else {
+#pragma unroll
+    for (int k = -C; k <= C; ++k)
+      acc = acc + (D != 2 ? tab[A.row * W + C + k] : (R)(ADJ ? O::dadj(A.row, C + k) : O::d(A.row, C + k))) * at(node_step(A, k, p.periodic));
+  }
+  return acc / (R)hdir(p, D);
+}
+template <typename R, int OPS, bool ADJ, typename I>
+__device__ __forceinline__ V3<R> line_derivs(const Params& p, int ix, int iy, int iz, const R* fx, const R* fy, const R* fz, I o, R* tab) {
+  const int per = p.periodic;
+  const NodeAxis ax = node_axis<OPS>(ix, p.nx, per), ay = node_axis<OPS>(iy, p.ny, per), az = node_axis<OPS>(iz, p.nz, per);
+  if (per || (az.mid && __all(ax.mid && ay.mid)))
+    return mk(line_deriv<R, OPS, ADJ, 0, true>(p, ax, fx, o, tab), line_deriv<R, OPS, ADJ, 1, true>(p, ay, fy, o, tab),
+              line_deriv<R, OPS, ADJ, 2, true>(p, az, fz, o, tab));
+  return mk(line_deriv<R, OPS, ADJ, 0, false>(p, ax, fx, o, tab), line_deriv<R, OPS, ADJ, 1, false>(p, ay, fy, o, tab),
+            line_deriv<R, OPS, ADJ, 2, false>(p, az, fz, o, tab));
+}
+#define IEQ_RUN_PREAMBLE(OFF)                                                                                \
+  using O = Op<OPS>;                                                                                          \
+  __shared__ R tabs[4][(2 * O::NB + 1) * O::W];                                                               \
+  R* tab = tabs[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)];                                            \
+  const int linear = (int)(blockIdx.y * kRow + blockIdx.x);                                                   \
+  if (linear >= cg.blocks) return;                                                                            \
+  const int tile = xcd_tile(linear, cg.blocks), zt = tile / cg.segs;                                          \
+  using P = std::conditional_t<std::is_same_v<I, unsigned>, uint32_t, uint64_t>;                              \
+  const P jt = (P)(tile - zt * cg.segs) * 256 + threadIdx.x, gx = (P)cg.gx, j = min(jt, (P)cg.gxy - 1);       \
+  const int ix = (int)(j % gx) + (OFF), iy = (int)(j / gx) + (OFF), iz = zt + (OFF);                          \
+  const long long S = p.stride, nxy = (long long)p.nx * p.ny;                                                 \
+  const I o = ((I)ix + (I)p.nx * (I)iy) * (I)sizeof(R);                                                       \
+  (void)S;
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_div(Params p, ColumnGrid cg, const R* b, R* out, int off) {
+  IEQ_RUN_PREAMBLE(off)
+  const R* f = b + iz * nxy;
+  const V3<R> d = line_derivs<R, OPS, false>(p, ix, iy, iz, f, f + S, f + 2 * S, o, tab);
+  if (jt < (P)cg.gxy) node_st(out + iz * nxy, o, d.x + d.y + d.z);
+}
+template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_grad(Params p, ColumnGrid cg, const R* f, R* out) {
+  IEQ_RUN_PREAMBLE(0)
+  const R* fz = f + iz * nxy;
+  const V3<R> d = line_derivs<R, OPS, false>(p, ix, iy, iz, fz, fz, fz, o, tab);
+  R* q = out + iz * nxy;
+  if (jt < (P)cg.gxy) {
+    node_st(q, o, d.x);
+    node_st(q + S, o, d.y);
+    node_st(q + 2 * S, o, d.z);
+  }
+}
 // Partial sums of the squared SBP norm of div B (calc_div + norm2_S, kernel_operator.cl:98-155): the
 // divergence in REAL as calc_div stores it, weights, squares and sums in double, of a component below 2 GiB (its
 // caller's limit).  One partial per block, at
@@ -288,23 +357,34 @@ template <typename R, int OPS> __global__ __launch_bounds__(BX* BY) void k_lap(P
 }
 
 // projector_divcleaning (kernel_div_cleaning.cl:96-109): B +/- grad(phi), .xyz only
-template <typename R, int OPS, typename I> __global__ __launch_bounds__(256) void k_proj(Params p, ColumnGrid cg, R* b, const R* phi) {
+template <typename R, int OPS, bool ADJ, typename I> __global__ __launch_bounds__(256) void k_proj(Params p, ColumnGrid cg, R* b, const R* phi) {
+  IEQ_RUN_PREAMBLE(0)
+  const R* f = phi + iz * nxy;
+  R* q = b + iz * nxy;
+  const R vx = node_ld(q, o), vy = node_ld(q + S, o), vz = node_ld(q + 2 * S, o);
+  const V3<R> d = line_derivs<R, OPS, ADJ>(p, ix, iy, iz, f, f, f, o, tab);
+  const R sgn = ADJ ? R(-1) : R(1);
+  if (jt < (P)cg.gxy) {
+    node_st(q, o, vx + sgn * d.x);
+    node_st(q + S, o, vy + sgn * d.y);
+    node_st(q + 2 * S, o, vz + sgn * d.z);
+  }
+}
+
+template <typename R, int OPS, bool ADJ, typename I> __global__ __launch_bounds__(256) void k_proj_column(Params p, ColumnGrid cg, R* b, const R* phi) {
   IEQ_COLUMN_PREAMBLE(0)
-  auto apply = [&](auto adj, R sgn) {
-    Column<R, OPS, decltype(adj)::value, I> c;
-    c.init(p, ix, iy);
-    c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
-      const R* f = phi + iz * nxy;
-      R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
-      const R vx = node_ld(bx, c.o), vy = node_ld(by, c.o), vz = node_ld(bz, c.o);
-      const R dx = c.template dx<x.value>(p, f), dy = c.template dy<y.value>(p, f), dz = c.template dz<z.value>(p, f, iz);
-      node_st(bx, c.o, vx + sgn * dx);
-      node_st(by, c.o, vy + sgn * dy);
-      node_st(bz, c.o, vz + sgn * dz);
-    });
-  };
-  if (p.laplace == 2) apply(std::true_type{}, R(-1));
-  else apply(std::false_type{}, R(1));
+  const R sgn = ADJ ? R(-1) : R(1);
+  Column<R, OPS, ADJ, I> c;
+  c.init(p, ix, iy);
+  c.planes(p, z0, z1, [&](auto x, auto y, auto z, int iz) {
+    const R* f = phi + iz * nxy;
+    R *bx = b + iz * nxy, *by = bx + S, *bz = by + S;
+    const R vx = node_ld(bx, c.o), vy = node_ld(by, c.o), vz = node_ld(bz, c.o);
+    const R dx = c.template dx<x.value>(p, f), dy = c.template dy<y.value>(p, f), dz = c.template dz<z.value>(p, f, iz);
+    node_st(bx, c.o, vx + sgn * dx);
+    node_st(by, c.o, vy + sgn * dy);
+    node_st(bz, c.o, vz + sgn * dz);
+  });
 }
 
 // calc_axpy (x = a x + y) / calc_xpay (x = x + a y), kernel_CG.cl:8-30
@@ -399,8 +479,30 @@ dim3 grid_of(Range g) { return dim3((g.x + BX - 1) / BX, (g.y + BY - 1) / BY, g.
     default: { constexpr int OPS = 5; CALL; } break; \
   }
 
-#define IEQ_PLANE_SWITCH(R, p, CALL) \
-  if (wide_plane<R>(p)) { using I = long long; CALL } else { using I = unsigned; CALL }
+// Whether the column kernels run an operator, or a thread per node.  A column finds the rows of a thread's nodes once and
+// runs whole planes without a branch, but holds the rows in registers, and on a wave that touches a face takes general
+// rows for all its lanes.  Columns / thread per node, us: FP32 bounded, div: 4th order 192^3 33 / 49, 256^3 62 / 109; 6th
+// extended 1000 x 8 x 200 42 / 21, 500 x 500 x 8 49 / 27; FP64 div: 2nd order 192^3 35 / 42, 4th 1000 x 8 x 200 36 / 19; 6th 128^3 56 / 33,
+// 256^3 482 / 254; projection, 6th extended, 1000 x 8 x 200 127 / 38.  Below 1.8 M nodes they are alike or the thread wins.
+template <typename R, int OPS> constexpr bool has_columns() { return sizeof(R) == 4 || Op<OPS>::W <= 7; }
+bool columns_pay(const Params& p) { return std::min(p.ny, p.nz) >= 32 && (long long)p.nx * p.ny * p.nz >= 1800000; }
+
+#define IEQ_COLUMN_SWITCH(R, p, ops, g, COLUMN, NODE)                \
+  const bool wide = wide_plane<R>(p), columns = columns_pay(p);      \
+  IEQ_OPS_SWITCH(ops, {                                              \
+    bool done = false;                                               \
+    if constexpr (has_columns<R, OPS>()) {                           \
+      if (columns) {                                                 \
+        const ColumnGrid cg = column_grid(g, 16);                    \
+        if (wide) { using I = long long; COLUMN; }                   \
+        else { using I = unsigned; COLUMN; }                         \
+        done = true;                                                 \
+      }                                                              \
+    }                                                                \
+    const ColumnGrid cg = column_grid(g, 1);                         \
+    if (!done && wide) { using I = long long; NODE; }                \
+    else if (!done) { using I = unsigned; NODE; }                    \
+  })
 
 template <typename R>
 void gen_update_2r(const Params& p, hipStream_t s, const uint32_t g[3], R* X, R* O, const R* D, R a, R b, R* time, double tc) {
@@ -429,8 +531,8 @@ template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32
 }
 
 template <typename R> void gen_div(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out, int off) {
-  const ColumnGrid cg = column_grid(g);
-  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_div<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out, off))))
+  IEQ_COLUMN_SWITCH(R, p, ops, g, (k_div_column<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out, off)),
+                    (k_div<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, out, off)))
 }
 
 template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s, const R* b, double* part, double* out) {
@@ -442,8 +544,8 @@ template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s
 }
 
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
-  const ColumnGrid cg = column_grid(g);
-  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_grad<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, f, out))))
+  IEQ_COLUMN_SWITCH(R, p, ops, g, (k_grad_column<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, f, out)),
+                    (k_grad<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, f, out)))
 }
 
 template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out) {
@@ -452,8 +554,13 @@ template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, cons
 }
 
 template <typename R> void gen_proj(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* b, const R* phi) {
-  const ColumnGrid cg = column_grid(g);
-  IEQ_PLANE_SWITCH(R, p, IEQ_OPS_SWITCH(ops, (k_proj<R, OPS, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi))))
+  if (p.laplace == 2) {
+    IEQ_COLUMN_SWITCH(R, p, ops, g, (k_proj_column<R, OPS, true, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi)),
+                      (k_proj<R, OPS, true, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi)))
+  } else {
+    IEQ_COLUMN_SWITCH(R, p, ops, g, (k_proj_column<R, OPS, false, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi)),
+                      (k_proj<R, OPS, false, I><<<cg.rows(), 256, 0, s>>>(p, cg, b, phi)))
+  }
 }
 
 template <typename R> void gen_axpy(const Params& p, hipStream_t s, const uint32_t g[3], R* x, const R* y, const R* a, int xpay) {

@@ -64,3 +64,19 @@ def test_curl_and_velocity_equal_oracle(ops, n, per, real, part):
                 assert _relerr(prog.download_real4(dev[k])[: cfg.num_nodes, :3], host[k][: cfg.num_nodes, :3]) <= tol, (lst, name)
             else:
                 assert bool((dev[k] == (3.0 if k == 3 else 2.0)).all())
+
+
+@pytest.mark.parametrize("ops,n,per,real", [
+    ("6thOrder", (130, 120, 118), False, "float"),          # columns, z-chunks of 1; boundary rows in most x waves
+    ("2ndOrderExtended", (200, 90, 101), False, "double"),  # columns
+    ("4thOrder", (128, 64, 230), True, "double"),           # columns, periodic
+    ("6thOrderExtended", (130, 120, 118), False, "double"),  # a thread per node: wide rows in FP64
+    ("4thOrder", (300, 230, 31), False, "float"),           # ... and few planes
+    ("6thOrder", (257, 13, 14), False, "float"),
+    ("2ndOrder", (9, 85, 12), True, "float"),
+])
+@pytest.mark.parametrize("part", [False, True])
+def test_operators_on_both_sides_of_the_column_rule(ops, n, per, real, part):
+    from test_gpu_node import test_column_kernels_equal_oracle as check
+
+    check(ops, n, per, real, part)

@@ -242,7 +242,8 @@ def test_planes_of_4_gib_take_64_bit_offsets(hip, real, below, above):
 
 @pytest.mark.parametrize("n", [(65600, 65600, 2), (1024, 1024, 1024), (100, 90, 80)])
 def test_column_kernels_launch_shape(hip, n):
-    """Runs of 256 nodes of a plane times z-chunks, in rows that HIP takes (4.3e9 nodes a plane: 1.7e7 runs)."""
+    """Runs of 256 nodes of a plane times planes or z-chunks, in rows that HIP takes (4.3e9 nodes a plane: 1.7e7
+    runs)."""
     hostrun(hip, """
         n = %r
         h = build(real="float", opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], testcase="rotation_2D", laplace="WIDE_STENCIL_LNS")
@@ -252,7 +253,8 @@ def test_column_kernels_launch_shape(hip, n):
             (l,) = log("launch", "refused")
             x, y, z, threads = [int(v) for v in l[2:6]]
             runs = (n[0] * n[1] + 255) // 256
-            zc = max(1, min(16, runs * n[2] // 4096))
+            zc = max(1, min(16, runs * n[2] // 4096)) if "column" in l[1] else 1
+            assert ("column" in l[1]) == (n == (1024, 1024, 1024))
             need = runs * -(-n[2] // zc)
             assert z == 1 and threads == 256 and need <= x * y < need + x, (x, y, need)
     """ % (n,))
