@@ -231,10 +231,7 @@ __device__ __forceinline__ R line_deriv(const Params& p, const NodeAxis& A, cons
   constexpr int W = O::W, C = (W - 1) / 2, NB = O::NB;
   const long long nxy = (long long)p.nx * p.ny;
   const bool mid = MID || (D == 2 ? A.mid : (bool)__all(A.mid));
-  if (D != 2 && !mid) {
-    for (int i = (int)threadIdx.x & 63; i < (2 * NB + 1) * W; i += 64) tab[i] = (R)(ADJ ? O::dadj(0, i) : O::d(0, i));
-    __builtin_amdgcn_wave_barrier();
-  }
+  if (D != 2 && !mid) wave_table<R, OPS, ADJ>(tab);
   R acc = R(0);
   auto at = [&](int step) {
     return D == 2 ? node_ld(f + (long long)step * nxy, o) : node_ld(f, o + (D == 0 ? (I)step : (I)step * (I)p.nx) * (I)sizeof(R));

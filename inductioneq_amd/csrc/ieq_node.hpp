@@ -56,7 +56,16 @@ template <typename T, int OPS, typename At> __device__ __forceinline__ T node_de
     if (k != 0) acc = acc + (T)O::d(O::NB, C + k) * at(k);
   return acc;
 }
-// The same for any row of the table, from its copy in LDS (a row differs from lane to lane: global
+// A wave's own copy of the derivative table (ADJ: of the adjoint's) in LDS, written and then read by its lanes: the
+// fences order the two without a workgroup barrier.
+template <typename R, int OPS, bool ADJ> __device__ __forceinline__ void wave_table(R* tab) {
+  using O = Op<OPS>;
+  for (int i = (int)threadIdx.x & 63; i < (2 * O::NB + 1) * O::W; i += 64) tab[i] = (R)(ADJ ? O::dadj(0, i) : O::d(0, i));
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+// The derivative for any row of the table, from a block's copy in LDS (a row differs from lane to lane: global
 // loads of it cost as much as the values it weighs, and registers for it cost occupancy).
 template <typename T, int OPS> struct NodeTable {
   static constexpr int W = Op<OPS>::W, C = (W - 1) / 2, ROWS = 2 * Op<OPS>::NB + 1;
