@@ -18,6 +18,9 @@ pytestmark = pytest.mark.gpu
     ("2ndOrderExtended", (70, 66, 20), False, "double"),
     ("4thOrder", (16, 16, 9), False, "double"),           # one block a plane
     ("4thOrder", (130, 40, 9), False, "float"),
+    ("4thOrder", (130, 40, 30), False, "float"),          # 156 k nodes: a thread per node, beyond it
+    ("4thOrder", (90, 85, 60), False, "double"),          # 459 k
+    ("2ndOrder", (90, 50, 41), True, "double"),           # 184 k
     ("6thOrder", (200, 20, 14), False, "double"),         # directions on waves of their own
     ("6thOrder", (200, 20, 14), False, "float"),
     ("6thOrderExtended", (20, 130, 17), False, "double"),

@@ -226,7 +226,7 @@ def test_planes_of_4_gib_take_64_bit_offsets(hip, real, below, above):
     """In-plane byte offsets of 32 bits wrap where a component's plane takes 4 GiB: kernels with 64-bit offsets there."""
     hostrun(hip, """
         names = {}
-        for n in (%r, %r, (64, 64, 9)):
+        for n in (%r, %r, (300, 300, 9)):
             h = build(real=%r, opset="4thOrder", nx=n[0], ny=n[1], nz=n[2], hall=True, testcase="hall_periodic",
                       laplace="WIDE_STENCIL_LNS")
             H.host_hip_clear()
