@@ -464,8 +464,9 @@ template <typename R> constexpr int hall_pd() { return sizeof(R) == 8 ? IEQ_HALL
 #endif
 
 // Waves per SIMD the single-grid kernel is compiled for.  FP64 holds two, except half-width 2 without convection in
-// the three-register forms, which fits three (4th order SSPRK33, HO dissipation: 128^3 51.2 -> 45.9 us a stage, 192^3
-// 168 -> 145); with the 2N update (48.8 -> 52.2) or convection (47.7 -> 65.9) a third wave spills.
+// the three-register forms, which fits three: it costs nothing where chunks are for two workgroups a CU (4th order SSPRK33,
+// HO dissipation, 128^3 42.3 and 42.4 us a stage, 200^3 158.7 and 159.2) and lets a third be resident where that pays
+// (pick_zc_hall: 144^3 58.2 -> 53.2).  With the 2N update (48.8 -> 52.2) or convection (47.7 -> 65.9) a third wave spills.
 template <typename R, int RR, bool CONV, int MODE> constexpr int hall_waves() {
   return sizeof(R) == 4 ? IEQ_HALL_WAVES32 : RR == 2 && !CONV && MODE >= 2 ? 3 : IEQ_HALL_WAVES;
 }
