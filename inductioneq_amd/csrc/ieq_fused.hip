@@ -272,13 +272,21 @@ bool brick_pays(int rr, int real_bytes, int nx, int ny, int nz) {
 // The EMF and stage brick kernels instead of k_hall_stage, which needs no E in memory but chains the planes of
 // both.  One kernel / bricks, us a stage (2N; SSPRK33 gains about 2 us more): FP32 half-width 3: 48^3 15.7 / 10.4, 96^3
 // 28.5 / 20.8, 120^3 39.2 / 37.3, 128^3 39.3 / 39.8 (with convection 96^3 34.4 / 23.0, 128^3 49.7 / 43.2, 160^3 82.4 / 86.4); 2:
-// 48^3 12.1 / 9.4, 96^3 20.8 / 18.5, 112^3 28.2 / 27.6, 128^3 30.5 / 36.1; 1: 48^3 9.2 / 8.7, 96^3 15.9 / 16.7.  FP64 half-width 3:
-// 48^3 19.7 / 15.1, 88^3 36.9 / 31.4, 96^3 36.9 / 37.2, 104^3 46.2 / 49.5 (with convection 96^3 45.9 / 43.4, 104^3 57.0 / 59.5); 2:
-// 64^3 15.5 / 16.4; 1: 64^3 10.7 / 14.5.  On the smallest grids of half-width 2 the second launch costs what is won.
-static bool brick_beats_hall(int rr, int real_bytes, bool conv, int nx, int ny, int nz) {
+// 48^3 12.1 / 9.4, 96^3 19.9 / 17.9, 100^3 24.1 / 24.7, without dissipation 104^3 24.5 / 21.7, 128^3 27.6 / 32.9; 1: 48^3 9.2 / 8.7, 96^3 15.9 / 16.7.
+// FP64 half-width 3: 48^3 19.7 / 15.1, 88^3 36.9 / 31.4, 96^3 36.9 / 39.0 (SSPRK33 34.3 / 33.7), 160 x 80 x 64 37.2 / 40.4, 90^3 37.8 /
+// 36.0 where the one kernel's 16 x 16 tiles have idle lanes; with convection 96^3 45.9 / 44.4, 128 x 96 x 90 53 / 56 (SSPRK33 47 / 43),
+// and without dissipation 96^3 38.0 / 39.8 (SSPRK33 35.3 / 34.7, 128 x 96 x 90 40 / 42.7); 2: 64^3 15.5 / 16.4; 1: 64^3 10.7 / 14.5.  On the
+// smallest grids of half-width 2 the second launch costs what is won.  A single step from an idle device (its launches are the
+// host's) is within 10 % of the one kernel's either way at 40^3 and faster elsewhere.
+static bool brick_beats_hall(int rr, int real_bytes, bool conv, bool hod, bool two_n, int nx, int ny, int nz) {
   const double n = (double)brick_nodes(nx, ny, nz);
-  if (rr == 3) return n <= (real_bytes == 4 ? (conv ? 3e6 : 1.9e6) : conv ? 1.2e6 : 0.9e6);
-  return rr == 2 && real_bytes == 4 && n >= 6e4 && n <= 1.5e6;
+  if (rr == 2) return real_bytes == 4 && n >= 6e4 && n <= (two_n && (hod || conv) ? 1.2e6 : 1.5e6);
+  if (rr != 3) return false;
+  if (real_bytes == 4) return n <= (conv ? 3e6 : 1.9e6);
+  if (!two_n) return n <= (!conv ? 0.9e6 : hod ? 1.2e6 : 1e6);
+  if (hod == conv) return n <= 0.9e6;
+  const double lanes = (double)((nx + 15) / 16 * 16) * ((ny + 15) / 16 * 16) / ((double)nx * ny);
+  return n <= 0.72e6 || (n <= 0.87e6 && lanes >= 1.04);
 }
 
 int hall_shape_for(long long nx, long long ny, long long nz, int real_bytes) {
@@ -546,7 +554,7 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
   bool forced = false;
   for (const char* k : {"IEQ_FUSED_TY", "IEQ_FUSED_ZC", "IEQ_EMF_ZC", "IEQ_FUSED_SPLIT", "IEQ_HALL_TILE"}) forced = forced || getenv(k);
   const bool moving = mn[0] != 0.0 || mn[1] != 0.0 || mn[2] != 0.0;
-  const bool brick = env_int("IEQ_BRICK", !forced && (p.hall ? brick_beats_hall(rr, sizeof(R), moving, p.nx, p.ny, p.nz)
+  const bool brick = env_int("IEQ_BRICK", !forced && (p.hall ? brick_beats_hall(rr, sizeof(R), moving, p.diss != 0, nf == 2, p.nx, p.ny, p.nz)
                                                              : brick_pays(rr, sizeof(R), p.nx, p.ny, p.nz)));
   const int ty = brick ? kBrickShape : ty_env == 4 || ty_env == 32 ? ty_env : 8;
   a.S = info.stride;
