@@ -722,7 +722,7 @@ int adjoint_create(const Params& p, const ieq_program_info& info, long long nste
   const bool narrow = info.real_bytes == 4 && p.nx % 64 != 0;
   A->ty = info.real_bytes == 8 ? 4 : 8;
   A->pre_tx = narrow ? 32 : 64;
-  A->shape = brick_pays(A->rr, info.real_bytes, p.nx, p.ny, p.nz) ? kBrickShape : info.real_bytes == 8 || narrow ? 32 : 8;
+  A->shape = brick_fits(info.stride, info.real_bytes) && brick_pays(A->rr, info.real_bytes, p.nx, p.ny, p.nz) ? kBrickShape : info.real_bytes == 8 || narrow ? 32 : 8;
   if (A->shape != kBrickShape) {
     int fake[3];  // distinct addresses standing for b1, b2, E: only compared, never read
     if (info.real_bytes == 8) {

@@ -554,7 +554,7 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
   bool forced = false;
   for (const char* k : {"IEQ_FUSED_TY", "IEQ_FUSED_ZC", "IEQ_EMF_ZC", "IEQ_FUSED_SPLIT", "IEQ_HALL_TILE"}) forced = forced || getenv(k);
   const bool moving = mn[0] != 0.0 || mn[1] != 0.0 || mn[2] != 0.0;
-  const bool brick = env_int("IEQ_BRICK", !forced && (p.hall ? brick_beats_hall(rr, sizeof(R), moving, p.diss != 0, nf == 2, p.nx, p.ny, p.nz)
+  const bool brick = brick_fits(info.stride, sizeof(R)) && env_int("IEQ_BRICK", !forced && (p.hall ? brick_beats_hall(rr, sizeof(R), moving, p.diss != 0, nf == 2, p.nx, p.ny, p.nz)
                                                              : brick_pays(rr, sizeof(R), p.nx, p.ny, p.nz)));
   const int ty = brick ? kBrickShape : ty_env == 4 || ty_env == 32 ? ty_env : 8;
   a.S = info.stride;

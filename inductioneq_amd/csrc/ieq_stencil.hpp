@@ -227,6 +227,8 @@ bool fused_plan(const std::string& I, int hall, std::vector<StageSpec>& v, int& 
 constexpr int kBrickShape = 1;
 template <typename R> void launch_emf(int rr, int ty, const FArgs<R>& a, hipStream_t s);
 template <typename R> void launch_stage(int rr, int ty, const FArgs<R>& a, bool hall, bool hod, hipStream_t s);
+// A brick's halo offsets are 32-bit and reach from the first component into the second (ieq_brick.hpp).
+inline bool brick_fits(long long stride, long long rb) { return stride * rb <= (1LL << 31); }
 // Whether the EMF and stage kernels run with a workgroup per brick of nodes rather than as z-marches.
 bool brick_pays(int rr, int real_bytes, int nx, int ny, int nz);
 template <typename R> void brick_emf(int rr, const FArgs<R>& a, hipStream_t s);

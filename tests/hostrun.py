@@ -22,7 +22,7 @@ P = ctypes.c_void_p
 
 
 def build(**kw):
-    cfg = ProgramConfig(w_size=64, **kw)
+    cfg = ProgramConfig(**{"w_size": 64, **kw})
     h, mods = P(), cfg.modules()
     arr = (ctypes.c_char_p * len(mods))(*[m.encode() for m in mods])
     assert lib.ieq_program_build(ctypes.byref(h), cfg.settings_string().encode(), arr, len(mods)) == 0, lib.ieq_last_error(None)

@@ -258,3 +258,22 @@ def test_column_kernels_launch_shape(hip, n):
             need = runs * -(-n[2] // zc)
             assert z == 1 and threads == 256 and need <= x * y < need + x, (x, y, need)
     """ % (n,))
+
+
+@pytest.mark.parametrize("w_size,bricks", [(64, True), (1 << 28, True), (1 << 29, False)])
+def test_bricks_only_where_their_offsets_fit(hip, w_size, bricks):
+    """A brick reaches the second component by a 32-bit byte offset from the first: components of more than 2 GiB (here
+    by the padding to W_SIZE) keep the z-march."""
+    hostrun(hip, """
+        h = build(real="double", opset="6thOrder", nx=40, ny=40, nz=40, periodic=True, testcase="uniform_flow", w_size=%d)
+        assert lib.ieq_step_uniform(h, b"SSPRK33", 1, (ctypes.c_double * 3)(0.1, 0.2, 0.3), 1.0, (P * 7)(*far(7)), 7, None) == 0
+        stages = [l[1] for l in log("launch") if "stage" in l[1]]
+        assert len(stages) == 3 and all(("brick" in k) == bool(%d) for k in stages), stages
+        a = P()
+        assert lib.ieq_adjoint_create(ctypes.byref(a), h, 2, 1) == 0, lib.ieq_last_error(h)
+        H.host_hip_clear()
+        c = ctypes.c_double(0.0)
+        assert lib.ieq_adjoint_forward(a, P(1 << 42), P(2 << 42), 1.0, (ctypes.c_double * 3)(0.1, 0.2, 0.3), ctypes.byref(c)) == 0, lib.ieq_last_error(h)
+        stages = [l[1] for l in log("launch") if "stage" in l[1]]
+        assert stages and all(("brick" in k) == bool(%d) for k in stages), stages
+    """ % (w_size, bricks, bricks))
