@@ -39,6 +39,7 @@ struct UniformState {
 struct FusedWork {
   void* scratch = nullptr;  // one vector field: ping-pong register of the 2N schemes
   size_t scratch_bytes = 0;
+  bool scratch_zero = false;  // ... has been cleared
   UniformState* uniform = nullptr;  // result of the uniformity check, pinned
   unsigned long long* seen = nullptr;  // device: the last check that found a difference
   unsigned long long checks = 0;
@@ -154,6 +155,10 @@ __global__ __launch_bounds__(256) void k_uniform_check(const R* u, const R* rho,
   if (varies && atomicMax(seen, check) < check) __hip_atomic_store(&out->varies, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (blockIdx.x == 0)
     for (int c = 0; c < 4; ++c) __hip_atomic_store(&out->v[c], (double)v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <typename R> __global__ __launch_bounds__(256) void k_zero(R* f, long long n) {
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) f[i] = R(0);
 }
 
 // nsteps applications of calc_time_* (kernel_time_integrator.cl:42-82).
@@ -534,11 +539,17 @@ int fused_step_t(const Params& p, const ieq_program_info& info, hipStream_t s, F
     w->scratch = nullptr;
     w->scratch_bytes = 0;
     if (hipMalloc(&w->scratch, vbytes) != hipSuccess) return w->scratch = nullptr, err = "hipMalloc failed", IEQ_ERR_HIP;
-    // the kernels write nodes only, and the copy back to b1 takes what follows them along
-    if (hipMemsetAsync(w->scratch, 0, vbytes, s) != hipSuccess) return err = "memset failed", IEQ_ERR_HIP;
     w->scratch_bytes = vbytes;
+    w->scratch_zero = false;
   }
-  if (nf == 2 && !SharedUse::capturing(s) && !opt.shared->enter(s)) return err = "event wait failed", IEQ_ERR_HIP;
+  const bool captured = SharedUse::capturing(s);
+  if (nf == 2 && !captured && !opt.shared->enter(s)) return err = "event wait failed", IEQ_ERR_HIP;
+  if (nf == 2 && !w->scratch_zero) {
+    // The kernels write nodes only, and the copy back to b1 takes what follows them along.  A kernel, because a call
+    // that is being captured records it; such a call has not cleared anything yet.
+    k_zero<R><<<1024, 256, 0, s>>>((R*)w->scratch, 3 * info.stride);
+    w->scratch_zero = !captured;
+  }
 
   FArgs<R> a{};
   a.nx = p.nx;
