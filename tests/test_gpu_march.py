@@ -53,3 +53,60 @@ def test_split_hall_march_equals_oracle(ops, n, integrator, source, real):
     hb, _ = _oracle_steps(cfg, B0, integrator, 2, u, 1.25)
     e = _relerr(args[0][:, : cfg.num_nodes].double().cpu().numpy().T, hb[0][: cfg.num_nodes, :3].astype(np.float64))
     assert e <= TOL[real], e
+
+
+@pytest.mark.parametrize("zc", ["3", "32"])
+@pytest.mark.parametrize("ops", ["2ndOrder", "4thOrder", "6thOrder", "2ndOrderExtended", "4thOrderExtended", "6thOrderExtended"])
+@pytest.mark.parametrize("diss", [None, "HIGH_ORDER", "FIRST_ORDER"])
+@pytest.mark.parametrize("per,real", [(False, "double"), (False, "float"), (True, "double"), (True, "float")])
+def test_tiled_stage_kernel(ops, diss, per, real, zc):
+    """The z-marching stage kernel of the reference schedule (a stated z-chunk keeps it on small grids): every operator
+    set and dissipation, every flux form over the cases, bounded with SAT data and periodic with a velocity of time."""
+    from test_gpu_tiled import FORMS, OPSETS, _cfg, _check, _run_both
+
+    k = OPSETS.index(ops) + 3 * [None, "HIGH_ORDER", "FIRST_ORDER"].index(diss) + 2 * per + (real == "float")
+    cfg = _cfg(ops, (37, 21, 19), per, diss, FORMS[k % len(FORMS)], "alfven_periodic_2D" if per else "rotation_2D", real)
+    prog, db, hb, path = _run_both(cfg, "SSPRK33", variable_u=per, env={"IEQ_TILED_ZC": zc})
+    assert path == "tiled"
+    _check(cfg, prog, db, hb, "SSPRK33", "%s %s %s %s" % (ops, diss, per, real))
+
+
+@pytest.mark.parametrize("integrator", INTEGRATORS)
+@pytest.mark.parametrize("per", [False, True])
+def test_tiled_stage_kernel_in_every_integrator(integrator, per):
+    from test_gpu_tiled import FORMS, _cfg, _check, _run_both
+
+    cfg = _cfg("4thOrder", (40, 26, 22), per, None, FORMS[per], "alfven_periodic_2D" if per else "gaussian_rotation_3D", "double")
+    prog, db, hb, path = _run_both(cfg, integrator, variable_u=per, env={"IEQ_TILED_ZC": "5"})
+    assert path == "tiled"
+    _check(cfg, prog, db, hb, integrator, integrator)
+
+
+@pytest.mark.parametrize("real,n", [("double", (76, 75, 74)), ("float", (110, 106, 104))])
+def test_tiled_stage_kernel_where_the_rule_takes_it(real, n):
+    """Periodic grids of a few nodes more than the rule's bound (400 k FP64, 1.2 M FP32) against a thread per node, one
+    step: the same sums in another order, 1e-13 and 1e-6 of the largest value."""
+    import torch
+    from test_gpu_tiled import FORMS, _aos, _cfg, _fields
+
+    from inductioneq_amd.program import Program
+    from inductioneq_amd.schedules import rk_schedule
+
+    cfg = _cfg("6thOrder", n, True, "HIGH_ORDER", FORMS[3], "alfven_periodic_2D", real)
+    prog = Program(cfg)
+    names, nf = rk_schedule("SSPRK33", False, True)
+    B, U = _fields(cfg, 9)
+    import os
+
+    out = {}
+    for mode in ("0", "1"):
+        os.environ["IEQ_NO_TILED"] = mode
+        try:
+            regs = [prog.upload_real4(_aos(cfg, B))] + [prog.vector() for _ in range(nf - 1)]
+            prog.run(names, regs + [prog.vector(), prog.upload_real4(_aos(cfg, U)), prog.scalar(1.0), prog.time_buffer(0.1)])
+            torch.cuda.synchronize()
+        finally:
+            os.environ.pop("IEQ_NO_TILED", None)
+        out[mode] = regs[0][:, : cfg.num_nodes].double()
+    e = float((out["0"] - out["1"]).abs().max() / out["1"].abs().max())
+    assert e <= (1e-13 if real == "double" else 1e-6), e
