@@ -78,7 +78,10 @@ const char *ieq_last_error(const ieq_program *prog);
 /* Parsed settings of a program. */
 int ieq_program_get_info(const ieq_program *prog, ieq_program_info *info);
 
-/* Stream on which all work of `prog` is enqueued (a hipStream_t; NULL = default stream). */
+/* Stream on which all work of `prog` is enqueued (a hipStream_t; NULL = default stream).  A call
+ * on the new stream that uses buffers the program keeps (2N stages) waits for the calls on the
+ * stream it leaves, which must not have been destroyed before; calls that are being captured do
+ * not, and the replays of their graphs are the caller's to order. */
 int ieq_set_stream(ieq_program *prog, void *hip_stream);
 
 /* Wait for all work enqueued on the program's stream. */
