@@ -281,8 +281,9 @@ bool brick_pays(int rr, int real_bytes, int nx, int ny, int nz) {
 // FP64 half-width 3: 48^3 19.7 / 15.1, 88^3 36.9 / 31.4, 96^3 36.9 / 39.0 (SSPRK33 34.3 / 33.7), 160 x 80 x 64 37.2 / 40.4, 90^3 37.8 /
 // 36.0 where the one kernel's 16 x 16 tiles have idle lanes; with convection 96^3 45.9 / 44.4, 128 x 96 x 90 53 / 56 (SSPRK33 47 / 43),
 // and without dissipation 96^3 38.0 / 39.8 (SSPRK33 35.3 / 34.7, 128 x 96 x 90 40 / 42.7); 2: 64^3 15.5 / 16.4; 1: 64^3 10.7 / 14.5.  On the
-// smallest grids of half-width 2 the second launch costs what is won.  A single step from an idle device (its launches are the
-// host's) is within 10 % of the one kernel's either way at 40^3 and faster elsewhere.
+// smallest grids of half-width 2 the second launch costs what is won.  One step from an idle device waits for the host's
+// launches, of which the bricks have twice as many: FP32 half-width 2, one kernel / bricks, 2N 40^3 76 / 83 us on one host
+// and 77 / 59 on another, SSPRK33 49 / 37; 64^3 2N 98 / 88; half-width 3, 16^3 to 48^3, 2N 91 to 95 / 64 to 68.
 static bool brick_beats_hall(int rr, int real_bytes, bool conv, bool hod, bool two_n, int nx, int ny, int nz) {
   const double n = (double)brick_nodes(nx, ny, nz);
   if (rr == 2) return real_bytes == 4 && n >= 6e4 && n <= (two_n && (hod || conv) ? 1.2e6 : 1.5e6);
