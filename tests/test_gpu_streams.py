@@ -79,3 +79,45 @@ def test_first_2n_list_while_another_stream_is_captured():
         return a[0].clone()
 
     assert torch.equal(solve(True), solve(False))
+
+
+def test_2n_steps_captured_between_eager_ones():
+    """2N steps on the default stream, then captured on another and replayed with eager steps on the first between the
+    replays: every replay gives what the same step gives eagerly."""
+    import torch
+    from test_gpu_fused import _device_args, _periodic_cfg
+
+    from inductioneq_amd.program import Program
+
+    u, rho = (0.3, -0.2, 0.1), 1.25
+    cfg = _periodic_cfg((40, 33, 26), "double", "6thOrder", True, "HIGH_ORDER", u, ho_factor=0.5)
+    B0 = np.asarray(random_modes_field((40, 33, 26), seed=4, kmax=2, amp=0.3))
+    cfg.dt = hall_dt(B0, (cfg.dx, cfg.dy, cfg.dz), 6, c_hall=0.8, cfl=0.3)
+    prog = Program(cfg)
+    step = lambda a: prog.step("CarpenterKennedy2N54", 3, a, uniform=(*u, rho))
+    inputs = [_device_args(prog, B0 * c, 2, u, rho)[0].clone() for c in (1.0, 0.7, 0.4)]
+    want = []
+    prog.use_current_stream()
+    for b in inputs:
+        a = _device_args(prog, B0, 2, u, rho)
+        a[0].copy_(b)
+        step(a)
+        torch.cuda.synchronize()
+        want.append(a[0].clone())
+    eager, captured, g = _device_args(prog, B0, 2, u, rho), _device_args(prog, B0, 2, u, rho), torch.cuda.CUDAGraph()
+    step(eager)
+    with torch.cuda.graph(g):
+        prog.use_current_stream()
+        step(captured)
+    prog.use_current_stream()
+    for k, b in enumerate(inputs):
+        captured[0].copy_(b)
+        captured[1].zero_()
+        captured[5].zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured[0], want[k]), k
+        eager[0].copy_(inputs[1])
+        step(eager)
+        torch.cuda.synchronize()
+        assert torch.equal(eager[0], want[1]), k
