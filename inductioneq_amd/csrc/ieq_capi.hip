@@ -185,7 +185,7 @@ struct ieq_program {
   double* diag = nullptr;  // ieq_diagnostics: 3 * kDiagBlocks partials + the 3 results
   // second copy of b1 for 2N stages that update it in the stage kernel (neighbours still read the first)
   void* b1_copy = nullptr;
-  ieq::SharedUse shared;  // of b1_copy and the fused steps' register
+  ieq::SharedUse shared;  // of b1_copy, the fused steps' register and the adjoint's registers and snapshots
 
   bool has(const char* m) const { return modules.count(m) != 0; }
   int fail(int code, const std::string& msg) {
@@ -543,6 +543,12 @@ bool args_apart(const ieq_program* pr, void* const* args, int nargs) {
     ++m;
   }
   return true;
+}
+
+// The call uses buffers of the program or of its adjoint on the present stream: ordered after their last use.
+int enter_shared(ieq_program* pr) {
+  if (ieq::SharedUse::capturing(pr->stream) || pr->shared.enter(pr->stream)) return IEQ_OK;
+  return pr->fail(IEQ_ERR_HIP, "event wait failed");
 }
 
 // Runs a kernel list.  Neighbouring kernels of the time integrators share a launch where every kernel of the
@@ -1124,11 +1130,13 @@ int ieq_adjoint_create(ieq_adjoint** adj, ieq_program* prog, long long nsteps, i
 
 int ieq_adjoint_forward(ieq_adjoint* adj, const void* b0, void* bT, double c_hall, const double u[3], double* kernel_seconds) {
   if (!adj || !b0 || !bT) return IEQ_ERR_ARGS;
+  if (int rc = enter_shared(adj->prog)) return rc;
   return ieq::adjoint_forward(adj->a, adj->prog->stream, b0, bT, c_hall, u, kernel_seconds, adj->prog->err);
 }
 
 int ieq_adjoint_backward(ieq_adjoint* adj, const void* lambda_T, void* grad_b0, double grads[4], double* kernel_seconds) {
   if (!adj || !lambda_T || !grad_b0 || !grads) return IEQ_ERR_ARGS;
+  if (int rc = enter_shared(adj->prog)) return rc;
   return ieq::adjoint_backward(adj->a, adj->prog->stream, lambda_T, grad_b0, grads, kernel_seconds, adj->prog->err);
 }
 

@@ -299,3 +299,21 @@ def test_fused_2n_register_is_cleared_by_a_kernel(hip):
         H.host_hip_capture(P(-1))
         assert step()[0] and not any(step())
     """)
+
+
+def test_adjoint_buffers_are_handed_from_stream_to_stream(hip):
+    """A forward solve on one stream and the backward on another: the second waits for the first's snapshots."""
+    hostrun(hip, """
+        h, a, c = build(opset="4thOrder", nx=16, ny=12, nz=12, periodic=True, hall=True, testcase="uniform_flow"), P(), ctypes.c_double(1.0)
+        bufs = [ctypes.create_string_buffer(3 * 2304 * 8) for _ in range(4)]
+        b = [ctypes.addressof(x) for x in bufs]
+        assert lib.ieq_set_stream(h, P(0x1000)) == 0
+        assert lib.ieq_adjoint_create(ctypes.byref(a), h, 3, 3) == 0, lib.ieq_last_error(h)
+        assert lib.ieq_adjoint_forward(a, P(b[0]), P(b[1]), 1.0, (ctypes.c_double * 3)(0.1, 0.2, 0.3), None) == 0, lib.ieq_last_error(h)
+        H.host_hip_clear()
+        assert lib.ieq_set_stream(h, P(0x2000)) == 0
+        assert lib.ieq_adjoint_backward(a, P(b[2]), P(b[3]), (ctypes.c_double * 4)(), None) == 0, lib.ieq_last_error(h)
+        kinds = [(l[0], l[1] if l[0] == "wait" else l[-1]) for l in log("wait", "record", "launch")]
+        assert kinds[:2] == [("record", "0x1000"), ("wait", "0x2000")], kinds[:4]
+        assert {k for k in kinds[2:]} <= {("record", "0x2000"), ("launch", "0x2000")}, kinds[:4]
+    """)
