@@ -485,6 +485,7 @@ int run_one(ieq_program* pr, const char* name, const uint32_t g[3], const uint32
     if ((rc = need("kernel_operator", 2))) return rc;
     if (!range_ok(pr, g, 0)) return pr->fail(IEQ_ERR_ARGS, n + ": NDRange exceeds the grid");
     if (n == "calc_curl") {
+      if (ieq::gen_curl<R>(p, ops, s, g, A(0), A(1))) return IEQ_OK;
       const hipError_t e = ieq::node_pre<R>(p, ops, s, g, A(0), A(1), (const R*)nullptr, (R*)nullptr, ieq::NodeTime<R>{});
       return e == hipSuccess ? IEQ_OK : hip_fail(pr, e, name);
     }

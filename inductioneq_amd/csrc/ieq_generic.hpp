@@ -18,6 +18,8 @@ template <typename R> void gen_init(const Params& p, hipStream_t s, const uint32
 template <typename R> void gen_div(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out, int off);
 // out[0] (device) = squared SBP norm of div B (calc_div + norm2_S); part: 1024 doubles of device scratch.
 template <typename R> void gen_div_norm2(const Params& p, int ops, hipStream_t s, const R* b, double* part, double* out);
+// False: not taken here (node_pre).
+template <typename R> bool gen_curl(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* b, R* out);
 template <typename R> void gen_grad(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out);
 template <typename R> void gen_lap(const Params& p, int ops, hipStream_t s, const uint32_t g[3], const R* f, R* out);
 template <typename R> void gen_proj(const Params& p, int ops, hipStream_t s, const uint32_t g[3], R* b, const R* phi);

@@ -25,6 +25,8 @@ pytestmark = pytest.mark.gpu
     ("6thOrder", (200, 20, 14), False, "float"),
     ("6thOrderExtended", (20, 130, 17), False, "double"),
     ("6thOrder", (130, 129, 110), False, "double"),       # 1.84 M nodes: a thread per node
+    ("2ndOrder", (130, 122, 118), False, "float"),        # columns
+    ("2ndOrderExtended", (200, 96, 99), False, "float"),
     ("6thOrder", (257, 9, 10), True, "float"),            # periodic: central rows only
     ("4thOrderExtended", (11, 93, 12), True, "double"),
 ])
@@ -77,6 +79,8 @@ def test_curl_and_velocity_equal_oracle(ops, n, per, real, part):
     ("4thOrder", (300, 230, 31), False, "float"),           # ... and few planes
     ("6thOrder", (257, 13, 14), False, "float"),
     ("2ndOrder", (9, 85, 12), True, "float"),
+    ("2ndOrder", (300, 31, 8), False, "float"),             # short rows in FP32: loaded together
+    ("2ndOrderExtended", (20, 19, 40), False, "float"),
 ])
 @pytest.mark.parametrize("part", [False, True])
 def test_operators_on_both_sides_of_the_column_rule(ops, n, per, real, part):
