@@ -7,6 +7,9 @@ first-order dissipation, bounded or periodic grids.  Each case runs whole RK ste
 reference RK_Step list) and checks that the tiled path ran.  Bar: FP64 1e-12 relative (max norm per
 register), FP32 2e-5 (1e-4 for work registers holding dt-scaled increments).  Grid sizes leave partial
 32 x 8 tiles; forced z-chunks of 2 and 5 planes put chunk boundaries next to the boundary planes.
+
+Below the sizes of its rule (tiled_stage_pays) the per-node kernel runs such stages and the path reads the same: the
+cases here without a stated z-chunk check that kernel, and test_gpu_march.py states one for every form of the tiled.
 """
 import math
 import os
